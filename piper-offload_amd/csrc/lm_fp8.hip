@@ -1,4 +1,5 @@
 // lm_fp8.hip -- scaled FP8 (TorchAO Float8Tensor) entry points.
+#include "lm_dequant.h"
 #include "lm_group.h"
 
 // ---------------------------------------------------------------------------
@@ -101,6 +102,12 @@ extern "C" int lm_fp8_dequant(const uint8_t* q, const float* scale, int64_t M, i
   if (!q || !scale || !out) return fail(LM_EINVAL, "FP8 dequant pointers must be non-null");
   if ((rc = check_fp8_layout(M, N, group, fp8_dtype))) return rc;
   if ((rc = check_lora(lora, M, N))) return rc;
+  if (!lora) {
+    if ((rc = check_dequant(M, N, out_dtype, workspace, workspace_bytes))) return rc;
+    DqArgs d{q, scale, nullptr, out, M, N, group, LM_F32, 0, {}};
+    if (fp8_dtype == LM_E4M3) return run_dequant<B_E4M3>(d, out_dtype, (hipStream_t)stream);
+    return run_dequant<B_E5M2>(d, out_dtype, (hipStream_t)stream);
+  }
   Ctx c;
   if ((rc = setup(c, M, N, lora, workspace, workspace_bytes, stream))) return rc;
   BlkArgs a = blk_args_base(c, M, N, lora, nullptr);
@@ -110,8 +117,7 @@ extern "C" int lm_fp8_dequant(const uint8_t* q, const float* scale, int64_t M, i
   a.group = group;
   a.out = out;
   a.out_dt = out_dtype;
-  const int cd = lora ? lora->dtype : (out_dtype == LM_F16 ? LM_F16 : LM_BF16);
-  if (fp8_dtype == LM_E4M3) return run_blocks<B_E4M3, P_TODENSE>(a, cd, c.nkc, false, false, c.st);
-  return run_blocks<B_E5M2, P_TODENSE>(a, cd, c.nkc, false, false, c.st);
+  if (fp8_dtype == LM_E4M3) return run_blocks<B_E4M3, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
+  return run_blocks<B_E5M2, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
 }
 

@@ -1690,6 +1690,13 @@ static inline int check_lora(const lm_lora* l, int64_t M, int64_t N) {
   return LM_OK;
 }
 
+static inline int check_workspace(const WsLayout& w, const void* ws, size_t wsb) {
+  if (!ws) return fail(LM_EWORKSPACE, "workspace pointer is null (need %zu bytes)", w.total);
+  if (wsb < w.total) return fail(LM_EWORKSPACE, "workspace too small: %zu < %zu bytes", wsb, w.total);
+  if (((uintptr_t)ws & 255) != 0) return fail(LM_EINVAL, "workspace must be 256-byte aligned");
+  return LM_OK;
+}
+
 // rows_split: the call runs the two-pass long-row kernels, whose row amax
 // slots the prep launch clears
 static inline int setup(Ctx& c, int64_t M, int64_t N, const lm_lora* l, void* ws, size_t wsb, void* stream,
@@ -1697,9 +1704,8 @@ static inline int setup(Ctx& c, int64_t M, int64_t N, const lm_lora* l, void* ws
   c.st = (hipStream_t)stream;
   const int rank = l ? l->rank : 0;
   WsLayout w = ws_layout(M, N, rank);
-  if (!ws) return fail(LM_EWORKSPACE, "workspace pointer is null (need %zu bytes)", w.total);
-  if (wsb < w.total) return fail(LM_EWORKSPACE, "workspace too small: %zu < %zu bytes", wsb, w.total);
-  if (((uintptr_t)ws & 255) != 0) return fail(LM_EINVAL, "workspace must be 256-byte aligned");
+  int rc;
+  if ((rc = check_workspace(w, ws, wsb))) return rc;
   uint8_t* base = (uint8_t*)ws;
   c.at = (uint16_t*)(base + w.at_off);
   c.bp = (uint16_t*)(base + w.bp_off);
@@ -1779,10 +1785,6 @@ static int run_blocks(const BlkArgs& a, int cd, int nkc, bool sr, bool from_dens
   if (from_dense) {
     if (sr) return run_blocks_cd<F, 1, true, true, PASS, false>(a, cd, st);
     return run_blocks_cd<F, 1, false, true, PASS, false>(a, cd, st);
-  }
-  if (nkc == 0) {
-    if (sr) return run_blocks_cd<F, 1, true, false, PASS, false>(a, cd, st);
-    return run_blocks_cd<F, 1, false, false, PASS, false>(a, cd, st);
   }
   if (sr) {
     NKC_SWITCH(nkc_bucket(nkc), return (run_blocks_cd<F, NKC_, true, false, PASS, true>(a, cd, st)));

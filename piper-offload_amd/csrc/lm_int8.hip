@@ -1,4 +1,5 @@
 // lm_int8.hip -- INT8 (TorchAO Int8Tensor) merge / requant / dequant entry points.
+#include "lm_dequant.h"
 #include "lm_group.h"
 
 // ---------------------------------------------------------------------------
@@ -109,6 +110,11 @@ extern "C" int lm_int8_dequant(const int8_t* q, const void* scale, const int8_t*
   if (!q || !scale || !out) return fail(LM_EINVAL, "INT8 dequant pointers must be non-null");
   if ((rc = check_int8_layout(M, N, group, scale_dtype))) return rc;
   if ((rc = check_lora(lora, M, N))) return rc;
+  if (!lora) {
+    if ((rc = check_dequant(M, N, out_dtype, workspace, workspace_bytes))) return rc;
+    DqArgs d{(const uint8_t*)q, scale, zero_point, out, M, N, group, scale_dtype, 0, {}};
+    return run_dequant<B_INT8>(d, out_dtype, (hipStream_t)stream);
+  }
   Ctx c;
   if ((rc = setup(c, M, N, lora, workspace, workspace_bytes, stream))) return rc;
   BlkArgs a = blk_args_base(c, M, N, lora, nullptr);
@@ -119,8 +125,7 @@ extern "C" int lm_int8_dequant(const int8_t* q, const void* scale, const int8_t*
   a.group = group;
   a.out = out;
   a.out_dt = out_dtype;
-  const int cd = lora ? lora->dtype : (out_dtype == LM_F16 ? LM_F16 : LM_BF16);
-  return run_blocks<B_INT8, P_TODENSE>(a, cd, c.nkc, false, false, c.st);
+  return run_blocks<B_INT8, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
 }
 
 

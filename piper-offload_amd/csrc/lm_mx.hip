@@ -1,4 +1,5 @@
 // lm_mx.hip -- MX (TorchAO MXTensor: MXFP4 / MXFP8) entry points.
+#include "lm_dequant.h"
 #include "lm_mx_fast.h"
 
 // ---------------------------------------------------------------------------
@@ -81,6 +82,13 @@ extern "C" int lm_mx_dequant(const uint8_t* q, const uint8_t* scale, int64_t M, 
   if (!q || !scale || !out) return fail(LM_EINVAL, "MX dequant pointers must be non-null");
   if ((rc = check_mx(M, N, elem_dtype, 0))) return rc;
   if ((rc = check_lora(lora, M, N))) return rc;
+  if (!lora) {
+    if ((rc = check_dequant(M, N, out_dtype, workspace, workspace_bytes))) return rc;
+    DqArgs d{q, scale, nullptr, out, M, N, N, LM_F32, swizzled, {}};
+    if (elem_dtype == LM_E2M1) return run_dequant<B_MXFP4>(d, out_dtype, (hipStream_t)stream);
+    if (elem_dtype == LM_E4M3) return run_dequant<B_MXE4M3>(d, out_dtype, (hipStream_t)stream);
+    return run_dequant<B_MXE5M2>(d, out_dtype, (hipStream_t)stream);
+  }
   Ctx c;
   if ((rc = setup(c, M, N, lora, workspace, workspace_bytes, stream))) return rc;
   BlkArgs a = blk_args_base(c, M, N, lora, nullptr);
@@ -89,7 +97,6 @@ extern "C" int lm_mx_dequant(const uint8_t* q, const uint8_t* scale, int64_t M, 
   a.swizzled = swizzled;
   a.out = out;
   a.out_dt = out_dtype;
-  const int cd = lora ? lora->dtype : (out_dtype == LM_F16 ? LM_F16 : LM_BF16);
-  return run_mx<P_TODENSE>(a, elem_dtype, cd, c.nkc, false, false, c.st);
+  return run_mx<P_TODENSE>(a, elem_dtype, lora->dtype, c.nkc, false, false, c.st);
 }
 

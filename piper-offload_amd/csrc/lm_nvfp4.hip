@@ -1,4 +1,5 @@
 // lm_nvfp4.hip -- NVFP4 (TorchAO NVFP4Tensor) entry points.
+#include "lm_dequant.h"
 #include "lm_nvfp4_fast.h"
 
 // ---------------------------------------------------------------------------
@@ -83,6 +84,11 @@ extern "C" int lm_nvfp4_dequant(const uint8_t* q, const uint8_t* scale, const fl
   if (!q || !scale || !out) return fail(LM_EINVAL, "NVFP4 dequant pointers must be non-null");
   if ((rc = check_nvfp4(M, N))) return rc;
   if ((rc = check_lora(lora, M, N))) return rc;
+  if (!lora) {
+    if ((rc = check_dequant(M, N, out_dtype, workspace, workspace_bytes))) return rc;
+    DqArgs d{q, scale, per_tensor_scale, out, M, N, N, LM_F32, swizzled, {}};
+    return run_dequant<B_NVFP4>(d, out_dtype, (hipStream_t)stream);
+  }
   Ctx c;
   if ((rc = setup(c, M, N, lora, workspace, workspace_bytes, stream))) return rc;
   BlkArgs a = blk_args_base(c, M, N, lora, nullptr);
@@ -92,7 +98,6 @@ extern "C" int lm_nvfp4_dequant(const uint8_t* q, const uint8_t* scale, const fl
   a.swizzled = swizzled;
   a.out = out;
   a.out_dt = out_dtype;
-  const int cd = lora ? lora->dtype : (out_dtype == LM_F16 ? LM_F16 : LM_BF16);
-  return run_blocks<B_NVFP4, P_TODENSE>(a, cd, c.nkc, false, false, c.st);
+  return run_blocks<B_NVFP4, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
 }
 

@@ -59,19 +59,6 @@ struct NvStackItem {
 
 constexpr int NV_NW = 8;
 
-// decode the two e2m1 codes of byte `b` of w to fp32 (low nibble -> .x).
-// The conversion's own scale operand stays 1.0: with a general bf16 block
-// scale it does not give the exact product (measured: the NVFP4 parity tests
-// fail), so the block scale is a separate multiply.
-DEV v2f32 e2m1_pair(uint32_t w, int b) {
-  switch (b) {
-    case 0: return __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0);
-    case 1: return __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
-    case 2: return __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2);
-    default: return __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
-  }
-}
-
 template <int NKC>
 struct NvTileIn {
   uint4 codes;
