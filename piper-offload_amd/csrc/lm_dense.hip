@@ -16,6 +16,6 @@ extern "C" int lm_dense_merge(void* w, int64_t M, int64_t N, int64_t ldw, const 
   a.q = w;
   a.q_out = w;
   a.ld = ldw;
-  return run_blocks<B_DENSE, P_FULL>(a, lora->dtype, c.nkc, false, false, c.st);
+  return run_blocks<B_DENSE, P_FULL>(a, lora->dtype, c.nkc, false, c.st);
 }
 

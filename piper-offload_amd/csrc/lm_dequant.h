@@ -16,26 +16,6 @@
 #pragma once
 #include "lm_impl.h"
 
-// n / d for every 32-bit n (Granlund and Montgomery, "Division by invariant
-// integers using multiplication", PLDI'94, figure 4.1)
-struct FastDiv {
-  uint32_t d, mul, sh1, sh2;
-};
-static inline FastDiv fast_div(uint32_t d) {
-  int l = 0;
-  while (l < 32 && (uint64_t(1) << l) < d) ++l;
-  FastDiv f;
-  f.d = d;
-  f.mul = (uint32_t)(((((uint64_t)1 << l) - d) << 32) / d + 1);
-  f.sh1 = l < 1 ? l : 1;
-  f.sh2 = l > 1 ? l - 1 : 0;
-  return f;
-}
-DEV uint32_t div_by(const FastDiv& f, uint32_t n) {
-  const uint32_t t = __umulhi(f.mul, n);
-  return (t + ((n - t) >> f.sh1)) >> f.sh2;
-}
-
 struct DqArgs {
   const uint8_t* q;
   const void* scale;

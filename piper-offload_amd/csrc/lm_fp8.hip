@@ -1,6 +1,7 @@
 // lm_fp8.hip -- scaled FP8 (TorchAO Float8Tensor) entry points.
 #include "lm_dequant.h"
 #include "lm_group.h"
+#include "lm_requant.h"
 
 // ---------------------------------------------------------------------------
 // FP8
@@ -16,19 +17,13 @@ static int check_fp8_layout(int64_t M, int64_t N, int64_t group, int32_t fmt) {
   return LM_OK;
 }
 
-static int fp8_common(const uint8_t* q, const float* scale, const void* dense, int dense_dt, uint8_t* q_out,
-                      float* scale_out, int64_t M, int64_t N, int64_t group, int32_t fmt, const lm_lora* lora,
-                      const lm_rounding* rnd, void* ws, size_t wsb, void* stream) {
+template <int KIND, int BF>
+static int fp8_merge(const uint8_t* q, const float* scale, uint8_t* q_out, float* scale_out, int64_t M, int64_t N,
+                     int64_t group, const lm_lora* lora, const lm_rounding* rnd, void* ws, size_t wsb, void* stream) {
   int rc;
-  if ((rc = check_fp8_layout(M, N, group, fmt))) return rc;
-  if ((rc = check_lora(lora, M, N))) return rc;
-  if ((rc = check_rounding(rnd))) return rc;
-  if (!q_out || !scale_out) return fail(LM_EINVAL, "FP8 outputs must be non-null");
-  const int cd = lora ? lora->dtype : dense_dt;
+  const int cd = lora->dtype;
   const bool sr = is_sr(rnd);
-  const bool split = !dense && group == N && lora &&
-                     rows_split_wanted(fmt == LM_E4M3 ? K_E4M3 : K_E5M2, cd, LM_F32, false, sr,
-                                       rpad_of(lora->rank) / 16, M, N);
+  const bool split = group == N && rows_split_wanted(KIND, cd, LM_F32, false, sr, rpad_of(lora->rank) / 16, M, N);
   Ctx c;
   if ((rc = setup(c, M, N, lora, ws, wsb, stream, split))) return rc;
   if (group == N || group != M * N) {  // per-row, or per-group
@@ -36,47 +31,36 @@ static int fp8_common(const uint8_t* q, const float* scale, const void* dense, i
     memset(&a, 0, sizeof a);
     a.q = q;
     a.scale = scale;
-    a.dense = (const uint16_t*)dense;
     a.q_out = q_out;
     a.scale_out = scale_out;
     a.at = c.at;
     a.bp = c.bp;
     a.M = M;
     a.N = N;
-    a.strength = lora ? lora->strength : 0.0f;
+    a.strength = lora->strength;
     a.seed = seed_of(rnd);
     a.red = split ? c.red : nullptr;
-    if (group != N) {
-      if (fmt == LM_E4M3) {
-        if (dense) return run_groups<K_E4M3, true>(a, group, cd, LM_F32, false, sr, 0, c.st);
-        return run_groups<K_E4M3, false>(a, group, cd, LM_F32, false, sr, c.nkc, c.st);
-      }
-      if (dense) return run_groups<K_E5M2, true>(a, group, cd, LM_F32, false, sr, 0, c.st);
-      return run_groups<K_E5M2, false>(a, group, cd, LM_F32, false, sr, c.nkc, c.st);
-    }
-    if (fmt == LM_E4M3) {
-      if (dense) return run_rows<K_E4M3, true>(a, cd, LM_F32, false, sr, 0, c.st);
-      return run_rows<K_E4M3, false>(a, cd, LM_F32, false, sr, c.nkc, c.st);
-    }
-    if (dense) return run_rows<K_E5M2, true>(a, cd, LM_F32, false, sr, 0, c.st);
-    return run_rows<K_E5M2, false>(a, cd, LM_F32, false, sr, c.nkc, c.st);
+    if (group != N) return run_groups<KIND, false>(a, group, cd, LM_F32, false, sr, c.nkc, c.st);
+    return run_rows<KIND, false>(a, cd, LM_F32, false, sr, c.nkc, c.st);
   }
   BlkArgs a = blk_args_base(c, M, N, lora, rnd);
   a.q = q;
   a.scale = scale;
-  a.dense = (const uint16_t*)dense;
   a.q_out = q_out;
   a.scale_out = scale_out;
   a.scale_dt = LM_F32;
   a.group = group;
-  if (fmt == LM_E4M3) {
-    if ((rc = run_blocks<B_E4M3, P_AMAX>(a, cd, c.nkc, false, dense != nullptr, c.st))) return rc;
-    if ((rc = run_blocks<B_E4M3, P_QUANT>(a, cd, c.nkc, sr, dense != nullptr, c.st))) return rc;
-    return run_finalize<B_E4M3>(a, cd, c.st) ? fail(LM_EHIP, "finalize launch failed") : LM_OK;
-  }
-  if ((rc = run_blocks<B_E5M2, P_AMAX>(a, cd, c.nkc, false, dense != nullptr, c.st))) return rc;
-  if ((rc = run_blocks<B_E5M2, P_QUANT>(a, cd, c.nkc, sr, dense != nullptr, c.st))) return rc;
-  return run_finalize<B_E5M2>(a, cd, c.st) ? fail(LM_EHIP, "finalize launch failed") : LM_OK;
+  if ((rc = run_blocks<BF, P_AMAX>(a, cd, c.nkc, false, c.st))) return rc;
+  if ((rc = run_blocks<BF, P_QUANT>(a, cd, c.nkc, sr, c.st))) return rc;
+  return run_finalize<BF>(a, cd, c.st) ? fail(LM_EHIP, "finalize launch failed") : LM_OK;
+}
+template <int KIND>
+static int fp8_requant(const RqArgs& r, int64_t group, int cd, bool sr, void* ws, hipStream_t st) {
+  if (group == r.M * r.N && group != r.N) return run_rq_tensor<KIND>(r, cd, false, sr, ws, st);
+  if (rq_rows_ok(r, group)) return run_rq_rows<KIND>(r, group, cd, false, sr, st);
+  RowArgs a = rq_row_args(r);
+  if (group != r.N) return run_groups<KIND, true>(a, group, cd, LM_F32, false, sr, 0, st);
+  return run_rows<KIND, true>(a, cd, LM_F32, false, sr, 0, st);
 }
 
 extern "C" int lm_fp8_merge(const uint8_t* q, const float* scale, uint8_t* q_out, float* scale_out, int64_t M, int64_t N,
@@ -84,16 +68,32 @@ extern "C" int lm_fp8_merge(const uint8_t* q, const float* scale, uint8_t* q_out
                             void* workspace, size_t workspace_bytes, void* stream) {
   if (!q || !scale) return fail(LM_EINVAL, "FP8 inputs must be non-null");
   if (!lora) return fail(LM_EINVAL, "lm_fp8_merge requires LoRA factors");
-  return fp8_common(q, scale, nullptr, 0, q_out, scale_out, M, N, group, fp8_dtype, lora, rounding, workspace,
-                    workspace_bytes, stream);
+  int rc;
+  if ((rc = check_fp8_layout(M, N, group, fp8_dtype))) return rc;
+  if ((rc = check_lora(lora, M, N))) return rc;
+  if ((rc = check_rounding(rounding))) return rc;
+  if (!q_out || !scale_out) return fail(LM_EINVAL, "FP8 outputs must be non-null");
+  if (fp8_dtype == LM_E4M3)
+    return fp8_merge<K_E4M3, B_E4M3>(q, scale, q_out, scale_out, M, N, group, lora, rounding, workspace, workspace_bytes,
+                                     stream);
+  return fp8_merge<K_E5M2, B_E5M2>(q, scale, q_out, scale_out, M, N, group, lora, rounding, workspace, workspace_bytes,
+                                   stream);
 }
 extern "C" int lm_fp8_requant(const void* dense, int32_t dense_dtype, uint8_t* q_out, float* scale_out, int64_t M,
                               int64_t N, int64_t group, int32_t fp8_dtype, const lm_rounding* rounding, void* workspace,
                               size_t workspace_bytes, void* stream) {
   if (!dense) return fail(LM_EINVAL, "dense input must be non-null");
   if (dense_dtype != LM_BF16 && dense_dtype != LM_F16) return fail(LM_EUNSUPPORTED, "requant input must be bf16/fp16");
-  return fp8_common(nullptr, nullptr, dense, dense_dtype, q_out, scale_out, M, N, group, fp8_dtype, nullptr, rounding,
-                    workspace, workspace_bytes, stream);
+  int rc;
+  if ((rc = check_fp8_layout(M, N, group, fp8_dtype))) return rc;
+  if ((rc = check_rounding(rounding))) return rc;
+  if (!q_out || !scale_out) return fail(LM_EINVAL, "FP8 outputs must be non-null");
+  if ((rc = check_workspace(ws_layout(M, N, 0), workspace, workspace_bytes))) return rc;
+  RqArgs r = rq_args(dense, q_out, scale_out, nullptr, M, N, rounding);
+  r.scale_dt = LM_F32;
+  if (fp8_dtype == LM_E4M3)
+    return fp8_requant<K_E4M3>(r, group, dense_dtype, is_sr(rounding), workspace, (hipStream_t)stream);
+  return fp8_requant<K_E5M2>(r, group, dense_dtype, is_sr(rounding), workspace, (hipStream_t)stream);
 }
 extern "C" int lm_fp8_dequant(const uint8_t* q, const float* scale, int64_t M, int64_t N, int64_t group, int32_t fp8_dtype,
                               const lm_lora* lora, void* out, int32_t out_dtype, void* workspace, size_t workspace_bytes,
@@ -117,7 +117,7 @@ extern "C" int lm_fp8_dequant(const uint8_t* q, const float* scale, int64_t M, i
   a.group = group;
   a.out = out;
   a.out_dt = out_dtype;
-  if (fp8_dtype == LM_E4M3) return run_blocks<B_E4M3, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
-  return run_blocks<B_E5M2, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
+  if (fp8_dtype == LM_E4M3) return run_blocks<B_E4M3, P_TODENSE>(a, lora->dtype, c.nkc, false, c.st);
+  return run_blocks<B_E5M2, P_TODENSE>(a, lora->dtype, c.nkc, false, c.st);
 }
 

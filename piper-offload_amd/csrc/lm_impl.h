@@ -16,8 +16,10 @@
 //                 workspace slots, then a pass that merges again and
 //                 quantizes, each over freely tiled 64-column tiles.
 //   k_blocks    : block-local formats (NVFP4 block 16, MX block 32, GGUF
-//                 Q8_0 block 32), dense bf16 weights, dequantize-to-dense,
-//                 and the two passes of per-tensor / two-level formats.
+//                 Q8_0 block 32), dense bf16 weights, merge-to-dense, and the
+//                 two passes of per-tensor / two-level formats.
+// Decode without a merge is in lm_dequant.h, encode of dense weights in
+// lm_requant.h.
 // Every element's delta comes from the same MFMA chain (tile_delta), so a
 // fused merge and the dense merge of the same inputs see identical values.
 #include <hip/hip_runtime.h>
@@ -292,6 +294,26 @@ struct TimedLaunch {
 // ---------------------------------------------------------------------------
 // shared argument blocks
 // ---------------------------------------------------------------------------
+// n / d for every 32-bit n (Granlund and Montgomery, "Division by invariant
+// integers using multiplication", PLDI'94, figure 4.1)
+struct FastDiv {
+  uint32_t d, mul, sh1, sh2;
+};
+static inline FastDiv fast_div(uint32_t d) {
+  int l = 0;
+  while (l < 32 && (uint64_t(1) << l) < d) ++l;
+  FastDiv f;
+  f.d = d;
+  f.mul = (uint32_t)(((((uint64_t)1 << l) - d) << 32) / d + 1);
+  f.sh1 = l < 1 ? l : 1;
+  f.sh2 = l > 1 ? l - 1 : 0;
+  return f;
+}
+DEV uint32_t div_by(const FastDiv& f, uint32_t n) {
+  const uint32_t t = __umulhi(f.mul, n);
+  return (t + ((n - t) >> f.sh1)) >> f.sh2;
+}
+
 enum RowKind : int { K_INT8 = 0, K_E4M3 = 1, K_E5M2 = 2 };
 
 struct RowArgs {
@@ -1221,7 +1243,6 @@ struct BlkArgs {
   const void* q;
   const void* scale;
   const void* aux;        // nvfp4: per-tensor scale in (float*); int8: zero point (int8*)
-  const uint16_t* dense;  // requant-only input
   void* q_out;
   void* scale_out;
   void* aux_out;          // nvfp4: per-tensor scale out; int8: zero point out
@@ -1521,7 +1542,35 @@ __device__ RowQP tensor_qparams(const BlkArgs& a, float& stored, int& zp) {
   }
 }
 
-template <int F, int CD, int NKC, bool SR, bool FROM_DENSE, int PASS, bool HAS_LORA>
+// a lane's SPAN dense values at flat offset o (left: elements to the row's
+// end), 16 bytes per store where the row and the output's alignment allow
+template <int SPAN>
+__device__ __forceinline__ void blk_store_dense(const BlkArgs& a, int64_t o, int64_t left, const float (&m)[SPAN]) {
+  if (left < SPAN || (a.N & 7) != 0 || ((uintptr_t)a.out & 15) != 0) {
+    for (int j = 0; j < SPAN && j < left; ++j) store_scalar(a.out, o + j, a.out_dt, m[j]);
+    return;
+  }
+  if (a.out_dt == BF16 || a.out_dt == F16) {
+    LM_GLOBAL lm_u32x4* p = (LM_GLOBAL lm_u32x4*)((LM_GLOBAL uint16_t*)a.out + o);
+#pragma unroll
+    for (int i = 0; i < SPAN / 8; ++i) {
+      lm_u32x4 w;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float lo = m[8 * i + 2 * k], hi = m[8 * i + 2 * k + 1];
+        w[k] = a.out_dt == BF16 ? pack_bf16x2(lo, hi) : (uint32_t)f16_bits(lo) | ((uint32_t)f16_bits(hi) << 16);
+      }
+      store_b128_guarded(p + i, w);
+    }
+  } else {
+    LM_GLOBAL lm_u32x4* p = (LM_GLOBAL lm_u32x4*)((LM_GLOBAL float*)a.out + o);
+#pragma unroll
+    for (int i = 0; i < SPAN / 4; ++i)
+      store_b128_guarded(p + i, lm_u32x4{f2u(m[4 * i]), f2u(m[4 * i + 1]), f2u(m[4 * i + 2]), f2u(m[4 * i + 3])});
+  }
+}
+
+template <int F, int CD, int NKC, bool SR, int PASS>
 __global__ __launch_bounds__(256) void k_blocks(BlkArgs a) {
   constexpr int SPAN = BlkTraits<F>::SPAN;
   constexpr int MTW = 4 * SPAN;
@@ -1559,7 +1608,7 @@ __global__ __launch_bounds__(256) void k_blocks(BlkArgs a) {
   if constexpr (F == B_NVFP4) gin = a.aux ? *(const float*)a.aux : 1.0f;
 
   v4i16 bop[NKC];
-  if constexpr (HAS_LORA && !FROM_DENSE) load_bop<NKC>(a.bp, active ? row : 0, lane, bop);
+  load_bop<NKC>(a.bp, active ? row : 0, lane, bop);
 
   float vmx = 0.0f, vmn = 0.0f;
   if (active) {
@@ -1568,32 +1617,20 @@ __global__ __launch_bounds__(256) void k_blocks(BlkArgs a) {
       if (mt >= ntiles) break;
       const int64_t mt_col0 = (int64_t)mt * MTW;
       const int64_t c0 = mt_col0 + SPAN * g;
-      float m[SPAN];
-      if constexpr (FROM_DENSE) {
+      float m[SPAN], base[SPAN], d[SPAN];
+      float auxv = 0.0f;
+      blk_load_base<F, CD>(a, row, rok, c0, gin, base, auxv);
+      tile_delta<SPAN, NKC, CD == F16>(a.at, mt_col0, lane, bop, d);
 #pragma unroll
-        for (int j = 0; j < SPAN; ++j) m[j] = (rok && c0 + j < N) ? val_dt<CD>(a.dense[row * N + c0 + j]) : 0.0f;
-      } else {
-        float base[SPAN];
-        float auxv = 0.0f;
-        blk_load_base<F, CD>(a, row, rok, c0, gin, base, auxv);
-        if constexpr (HAS_LORA) {
-          float d[SPAN];
-          tile_delta<SPAN, NKC, CD == F16>(a.at, mt_col0, lane, bop, d);
-#pragma unroll
-          for (int j = 0; j < SPAN; ++j) {
-            float v;
-            if constexpr (F == B_NVFP4) {
-              float upd = d[j] * a.strength;
-              v = (upd == 0.0f) ? base[j] : round_dt<CD>(__builtin_fmaf(d[j], a.strength, base[j]));
-            } else {
-              v = round_dt<CD>(__builtin_fmaf(d[j], a.strength, base[j]));
-            }
-            m[j] = (rok && c0 + j < N) ? v : 0.0f;
-          }
+      for (int j = 0; j < SPAN; ++j) {
+        float v;
+        if constexpr (F == B_NVFP4) {
+          float upd = d[j] * a.strength;
+          v = (upd == 0.0f) ? base[j] : round_dt<CD>(__builtin_fmaf(d[j], a.strength, base[j]));
         } else {
-#pragma unroll
-          for (int j = 0; j < SPAN; ++j) m[j] = base[j];
+          v = round_dt<CD>(__builtin_fmaf(d[j], a.strength, base[j]));
         }
+        m[j] = (rok && c0 + j < N) ? v : 0.0f;
       }
       if constexpr (PASS == P_AMAX) {
 #pragma unroll
@@ -1606,9 +1643,7 @@ __global__ __launch_bounds__(256) void k_blocks(BlkArgs a) {
           }
         }
       } else if constexpr (PASS == P_TODENSE) {
-        if (rok) {
-          for (int j = 0; j < SPAN && c0 + j < N; ++j) store_scalar(a.out, row * N + c0 + j, a.out_dt, m[j]);
-        }
+        if (rok && c0 < N) blk_store_dense<SPAN>(a, row * N + c0, N - c0, m);
       } else {
         if (rok && c0 < N) blk_store<F, CD, SR>(a, row, c0, m, gscale, gqp);
       }
@@ -1763,7 +1798,7 @@ static inline unsigned blocks_for(int64_t M, int64_t N, int mtw, int tpw) {
   return (unsigned)((units + 3) / 4);
 }
 
-template <int F, int NKC, bool SR, bool FROM_DENSE, int PASS, bool HAS_LORA>
+template <int F, int NKC, bool SR, int PASS>
 static int run_blocks_cd(const BlkArgs& a, int cd, hipStream_t st) {
   constexpr int SPAN = BlkTraits<F>::SPAN;
   unsigned nb = blocks_for(a.M, a.N, 4 * SPAN, a.tpw);
@@ -1772,24 +1807,20 @@ static int run_blocks_cd(const BlkArgs& a, int cd, hipStream_t st) {
                                                                                                     : "todense",
                     st);
   if (cd == LM_F16)
-    hipLaunchKernelGGL((k_blocks<F, F16, NKC, SR, FROM_DENSE, PASS, HAS_LORA>), dim3(nb), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_blocks<F, F16, NKC, SR, PASS>), dim3(nb), dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((k_blocks<F, BF16, NKC, SR, FROM_DENSE, PASS, HAS_LORA>), dim3(nb), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_blocks<F, BF16, NKC, SR, PASS>), dim3(nb), dim3(256), 0, st, a);
   LAUNCH_CHECK();
   return LM_OK;
 }
 
-// run a block kernel for the given pass with optional LoRA / SR
+// run a block kernel for the given pass
 template <int F, int PASS>
-static int run_blocks(const BlkArgs& a, int cd, int nkc, bool sr, bool from_dense, hipStream_t st) {
-  if (from_dense) {
-    if (sr) return run_blocks_cd<F, 1, true, true, PASS, false>(a, cd, st);
-    return run_blocks_cd<F, 1, false, true, PASS, false>(a, cd, st);
-  }
+static int run_blocks(const BlkArgs& a, int cd, int nkc, bool sr, hipStream_t st) {
   if (sr) {
-    NKC_SWITCH(nkc_bucket(nkc), return (run_blocks_cd<F, NKC_, true, false, PASS, true>(a, cd, st)));
+    NKC_SWITCH(nkc_bucket(nkc), return (run_blocks_cd<F, NKC_, true, PASS>(a, cd, st)));
   } else {
-    NKC_SWITCH(nkc_bucket(nkc), return (run_blocks_cd<F, NKC_, false, false, PASS, true>(a, cd, st)));
+    NKC_SWITCH(nkc_bucket(nkc), return (run_blocks_cd<F, NKC_, false, PASS>(a, cd, st)));
   }
   return LM_OK;
 }

@@ -1,6 +1,7 @@
 // lm_int8.hip -- INT8 (TorchAO Int8Tensor) merge / requant / dequant entry points.
 #include "lm_dequant.h"
 #include "lm_group.h"
+#include "lm_requant.h"
 
 // ---------------------------------------------------------------------------
 // INT8
@@ -17,76 +18,61 @@ static int check_int8_layout(int64_t M, int64_t N, int64_t group, int32_t scale_
   return LM_OK;
 }
 
-static int int8_common(const int8_t* q, const void* scale, const int8_t* zp, const void* dense, int dense_dt, int8_t* q_out,
-                       void* scale_out, int8_t* zp_out, int64_t M, int64_t N, int64_t group, int32_t sdt, int32_t asym,
-                       int32_t reduce_range, const lm_lora* lora, const lm_rounding* rnd, void* ws, size_t wsb,
-                       void* stream) {
+extern "C" int lm_int8_merge(const int8_t* q, const void* scale, const int8_t* zero_point, int8_t* q_out, void* scale_out,
+                             int8_t* zero_point_out, int64_t M, int64_t N, int64_t group, int32_t scale_dtype,
+                             int32_t asymmetric, int32_t reduce_range, const lm_lora* lora, const lm_rounding* rounding,
+                             void* workspace, size_t workspace_bytes, void* stream) {
   int rc;
-  if ((rc = check_int8_layout(M, N, group, sdt))) return rc;
+  if (!q || !scale) return fail(LM_EINVAL, "INT8 inputs must be non-null");
+  if (!lora) return fail(LM_EINVAL, "lm_int8_merge requires LoRA factors");
+  if (asymmetric && (!zero_point_out)) return fail(LM_EINVAL, "asymmetric INT8 merge requires a zero-point output");
+  if ((rc = check_int8_layout(M, N, group, scale_dtype))) return rc;
   if ((rc = check_lora(lora, M, N))) return rc;
-  if ((rc = check_rounding(rnd))) return rc;
+  if ((rc = check_rounding(rounding))) return rc;
   if (!q_out || !scale_out) return fail(LM_EINVAL, "INT8 outputs must be non-null");
-  const int cd = lora ? lora->dtype : dense_dt;
-  const bool sr = is_sr(rnd);
-  const bool split = !dense && group == N && lora &&
-                     rows_split_wanted(K_INT8, cd, sdt, asym != 0, sr, rpad_of(lora->rank) / 16, M, N);
+  const int cd = lora->dtype;
+  const bool sr = is_sr(rounding), asym = asymmetric != 0;
+  const bool split = group == N && rows_split_wanted(K_INT8, cd, scale_dtype, asym, sr, rpad_of(lora->rank) / 16, M, N);
   Ctx c;
-  if ((rc = setup(c, M, N, lora, ws, wsb, stream, split))) return rc;
+  if ((rc = setup(c, M, N, lora, workspace, workspace_bytes, stream, split))) return rc;
   const int qmin = reduce_range ? -64 : -128, qmax = reduce_range ? 63 : 127;
   if (group == N || group != M * N) {  // per-row, or per-group
     RowArgs a;
     memset(&a, 0, sizeof a);
     a.q = q;
     a.scale = scale;
-    a.zp = zp;
-    a.dense = (const uint16_t*)dense;
+    a.zp = zero_point;
     a.q_out = q_out;
     a.scale_out = scale_out;
-    a.zp_out = zp_out;
+    a.zp_out = zero_point_out;
     a.at = c.at;
     a.bp = c.bp;
     a.M = M;
     a.N = N;
-    a.strength = lora ? lora->strength : 0.0f;
+    a.strength = lora->strength;
     a.qmin = qmin;
     a.qmax = qmax;
-    a.seed = seed_of(rnd);
+    a.seed = seed_of(rounding);
     a.red = split ? c.red : nullptr;
-    if (group != N) {
-      if (dense) return run_groups<K_INT8, true>(a, group, cd, sdt, asym != 0, sr, 0, c.st);
-      return run_groups<K_INT8, false>(a, group, cd, sdt, asym != 0, sr, c.nkc, c.st);
-    }
-    if (dense) return run_rows<K_INT8, true>(a, cd, sdt, asym != 0, sr, 0, c.st);
-    return run_rows<K_INT8, false>(a, cd, sdt, asym != 0, sr, c.nkc, c.st);
+    if (group != N) return run_groups<K_INT8, false>(a, group, cd, scale_dtype, asym, sr, c.nkc, c.st);
+    return run_rows<K_INT8, false>(a, cd, scale_dtype, asym, sr, c.nkc, c.st);
   }
   // per-tensor: two passes
-  BlkArgs a = blk_args_base(c, M, N, lora, rnd);
+  BlkArgs a = blk_args_base(c, M, N, lora, rounding);
   a.q = q;
   a.scale = scale;
-  a.aux = zp;
-  a.dense = (const uint16_t*)dense;
+  a.aux = zero_point;
   a.q_out = q_out;
   a.scale_out = scale_out;
-  a.aux_out = zp_out;
-  a.scale_dt = sdt;
+  a.aux_out = zero_point_out;
+  a.scale_dt = scale_dtype;
   a.qmin = qmin;
   a.qmax = qmax;
-  a.asym = asym;
+  a.asym = asymmetric;
   a.group = group;
-  if ((rc = run_blocks<B_INT8, P_AMAX>(a, cd, c.nkc, false, dense != nullptr, c.st))) return rc;
-  if ((rc = run_blocks<B_INT8, P_QUANT>(a, cd, c.nkc, sr, dense != nullptr, c.st))) return rc;
+  if ((rc = run_blocks<B_INT8, P_AMAX>(a, cd, c.nkc, false, c.st))) return rc;
+  if ((rc = run_blocks<B_INT8, P_QUANT>(a, cd, c.nkc, sr, c.st))) return rc;
   return run_finalize<B_INT8>(a, cd, c.st) ? fail(LM_EHIP, "finalize launch failed") : LM_OK;
-}
-
-extern "C" int lm_int8_merge(const int8_t* q, const void* scale, const int8_t* zero_point, int8_t* q_out, void* scale_out,
-                             int8_t* zero_point_out, int64_t M, int64_t N, int64_t group, int32_t scale_dtype,
-                             int32_t asymmetric, int32_t reduce_range, const lm_lora* lora, const lm_rounding* rounding,
-                             void* workspace, size_t workspace_bytes, void* stream) {
-  if (!q || !scale) return fail(LM_EINVAL, "INT8 inputs must be non-null");
-  if (!lora) return fail(LM_EINVAL, "lm_int8_merge requires LoRA factors");
-  if (asymmetric && (!zero_point_out)) return fail(LM_EINVAL, "asymmetric INT8 merge requires a zero-point output");
-  return int8_common(q, scale, zero_point, nullptr, 0, q_out, scale_out, zero_point_out, M, N, group, scale_dtype,
-                     asymmetric, reduce_range, lora, rounding, workspace, workspace_bytes, stream);
 }
 
 extern "C" int lm_int8_requant(const void* dense, int32_t dense_dtype, int8_t* q_out, void* scale_out,
@@ -96,11 +82,22 @@ extern "C" int lm_int8_requant(const void* dense, int32_t dense_dtype, int8_t* q
   if (!dense) return fail(LM_EINVAL, "dense input must be non-null");
   if (dense_dtype != LM_BF16 && dense_dtype != LM_F16)
     return fail(LM_EUNSUPPORTED, "requant input must be bfloat16 or float16");
-  if ((N & 7) != 0 && group == N) {
-    // the dense fast path needs 16-byte rows; the masked path handles the rest
-  }
-  return int8_common(nullptr, nullptr, nullptr, dense, dense_dtype, q_out, scale_out, zero_point_out, M, N, group,
-                     scale_dtype, asymmetric, reduce_range, nullptr, rounding, workspace, workspace_bytes, stream);
+  int rc;
+  if ((rc = check_int8_layout(M, N, group, scale_dtype))) return rc;
+  if ((rc = check_rounding(rounding))) return rc;
+  if (!q_out || !scale_out) return fail(LM_EINVAL, "INT8 outputs must be non-null");
+  if ((rc = check_workspace(ws_layout(M, N, 0), workspace, workspace_bytes))) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  const bool sr = is_sr(rounding), asym = asymmetric != 0;
+  RqArgs r = rq_args(dense, (uint8_t*)q_out, scale_out, zero_point_out, M, N, rounding);
+  r.scale_dt = scale_dtype;
+  r.qmin = reduce_range ? -64 : -128;
+  r.qmax = reduce_range ? 63 : 127;
+  if (group == M * N && group != N) return run_rq_tensor<K_INT8>(r, dense_dtype, asym, sr, workspace, st);
+  if (rq_rows_ok(r, group)) return run_rq_rows<K_INT8>(r, group, dense_dtype, asym, sr, st);
+  RowArgs a = rq_row_args(r);
+  if (group != N) return run_groups<K_INT8, true>(a, group, dense_dtype, scale_dtype, asym, sr, 0, st);
+  return run_rows<K_INT8, true>(a, dense_dtype, scale_dtype, asym, sr, 0, st);
 }
 
 extern "C" int lm_int8_dequant(const int8_t* q, const void* scale, const int8_t* zero_point, int64_t M, int64_t N,
@@ -125,7 +122,7 @@ extern "C" int lm_int8_dequant(const int8_t* q, const void* scale, const int8_t*
   a.group = group;
   a.out = out;
   a.out_dt = out_dtype;
-  return run_blocks<B_INT8, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
+  return run_blocks<B_INT8, P_TODENSE>(a, lora->dtype, c.nkc, false, c.st);
 }
 
 

@@ -1,6 +1,7 @@
 // lm_mx.hip -- MX (TorchAO MXTensor: MXFP4 / MXFP8) entry points.
 #include "lm_dequant.h"
 #include "lm_mx_fast.h"
+#include "lm_requant.h"
 
 // ---------------------------------------------------------------------------
 // MX
@@ -13,10 +14,10 @@ static int check_mx(int64_t M, int64_t N, int32_t elem, int32_t scaling) {
   return LM_OK;
 }
 template <int PASS>
-static int run_mx(const BlkArgs& a, int elem, int cd, int nkc, bool sr, bool from_dense, hipStream_t st) {
-  if (elem == LM_E2M1) return run_blocks<B_MXFP4, PASS>(a, cd, nkc, sr, from_dense, st);
-  if (elem == LM_E4M3) return run_blocks<B_MXE4M3, PASS>(a, cd, nkc, sr, from_dense, st);
-  return run_blocks<B_MXE5M2, PASS>(a, cd, nkc, sr, from_dense, st);
+static int run_mx(const BlkArgs& a, int elem, int cd, int nkc, bool sr, hipStream_t st) {
+  if (elem == LM_E2M1) return run_blocks<B_MXFP4, PASS>(a, cd, nkc, sr, st);
+  if (elem == LM_E4M3) return run_blocks<B_MXE4M3, PASS>(a, cd, nkc, sr, st);
+  return run_blocks<B_MXE5M2, PASS>(a, cd, nkc, sr, st);
 }
 extern "C" int lm_mx_merge(uint8_t* q, uint8_t* scale, int64_t M, int64_t N, int32_t elem_dtype, int32_t scaling,
                            int32_t swizzled, const lm_lora* lora, const lm_rounding* rounding, void* workspace,
@@ -55,7 +56,7 @@ extern "C" int lm_mx_merge(uint8_t* q, uint8_t* scale, int64_t M, int64_t N, int
   a.scale_out = scale;
   a.swizzled = swizzled;
   a.mx_mode = scaling;
-  return run_mx<P_FULL>(a, elem_dtype, lora->dtype, c.nkc, is_sr(rounding), false, c.st);
+  return run_mx<P_FULL>(a, elem_dtype, lora->dtype, c.nkc, is_sr(rounding), c.st);
 }
 extern "C" int lm_mx_requant(const void* dense, int32_t dense_dtype, uint8_t* q_out, uint8_t* scale_out, int64_t M,
                              int64_t N, int32_t elem_dtype, int32_t scaling, int32_t swizzled, const lm_rounding* rounding,
@@ -64,16 +65,16 @@ extern "C" int lm_mx_requant(const void* dense, int32_t dense_dtype, uint8_t* q_
   if (!dense || !q_out || !scale_out) return fail(LM_EINVAL, "MX requant pointers must be non-null");
   if ((rc = check_mx(M, N, elem_dtype, scaling))) return rc;
   if ((rc = check_rounding(rounding))) return rc;
-  Ctx c;
-  if ((rc = setup(c, M, N, nullptr, workspace, workspace_bytes, stream))) return rc;
-  BlkArgs a = blk_args_base(c, M, N, nullptr, rounding);
-  a.dense = (const uint16_t*)dense;
-  a.q_out = q_out;
-  a.scale_out = scale_out;
+  if ((rc = check_workspace(ws_layout(M, N, 0), workspace, workspace_bytes))) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  RqArgs a = rq_args(dense, q_out, scale_out, nullptr, M, N, rounding);
   a.swizzled = swizzled;
   a.mx_mode = scaling;
-  if (swizzled && (rc = zero_swizzle_pad(scale_out, M, N / 32, c.st))) return rc;
-  return run_mx<P_FULL>(a, elem_dtype, dense_dtype, 0, is_sr(rounding), true, c.st);
+  if (swizzled && (rc = zero_swizzle_pad(scale_out, M, N / 32, st))) return rc;
+  const bool sr = is_sr(rounding);
+  if (elem_dtype == LM_E2M1) return run_rq_blocks<B_MXFP4>(a, dense_dtype, sr, workspace, st);
+  if (elem_dtype == LM_E4M3) return run_rq_blocks<B_MXE4M3>(a, dense_dtype, sr, workspace, st);
+  return run_rq_blocks<B_MXE5M2>(a, dense_dtype, sr, workspace, st);
 }
 extern "C" int lm_mx_dequant(const uint8_t* q, const uint8_t* scale, int64_t M, int64_t N, int32_t elem_dtype,
                              int32_t swizzled, const lm_lora* lora, void* out, int32_t out_dtype, void* workspace,
@@ -97,6 +98,6 @@ extern "C" int lm_mx_dequant(const uint8_t* q, const uint8_t* scale, int64_t M, 
   a.swizzled = swizzled;
   a.out = out;
   a.out_dt = out_dtype;
-  return run_mx<P_TODENSE>(a, elem_dtype, lora->dtype, c.nkc, false, false, c.st);
+  return run_mx<P_TODENSE>(a, elem_dtype, lora->dtype, c.nkc, false, c.st);
 }
 

@@ -1,5 +1,6 @@
 // lm_q8.hip -- GGUF Q8_0 merge / requant and GGUF dequant entry points.
 #include "lm_q8_fast.h"
+#include "lm_requant.h"
 
 // ---------------------------------------------------------------------------
 // GGUF Q8_0
@@ -34,7 +35,7 @@ extern "C" int lm_q8_0_merge(const uint8_t* packed, uint8_t* packed_out, int64_t
   BlkArgs a = blk_args_base(c, M, N, lora, rounding);
   a.q = packed;
   a.q_out = packed_out;
-  return run_blocks<B_Q8_0, P_FULL>(a, lora->dtype, c.nkc, is_sr(rounding), false, c.st);
+  return run_blocks<B_Q8_0, P_FULL>(a, lora->dtype, c.nkc, is_sr(rounding), c.st);
 }
 extern "C" int lm_q8_0_requant(const void* dense, int32_t dense_dtype, uint8_t* packed_out, int64_t M, int64_t N,
                                const lm_rounding* rounding, void* workspace, size_t workspace_bytes, void* stream) {
@@ -42,12 +43,9 @@ extern "C" int lm_q8_0_requant(const void* dense, int32_t dense_dtype, uint8_t* 
   if (!dense || !packed_out) return fail(LM_EINVAL, "Q8_0 requant pointers must be non-null");
   if ((rc = check_q8(M, N))) return rc;
   if ((rc = check_rounding(rounding))) return rc;
-  Ctx c;
-  if ((rc = setup(c, M, N, nullptr, workspace, workspace_bytes, stream))) return rc;
-  BlkArgs a = blk_args_base(c, M, N, nullptr, rounding);
-  a.dense = (const uint16_t*)dense;
-  a.q_out = packed_out;
-  return run_blocks<B_Q8_0, P_FULL>(a, dense_dtype, 0, is_sr(rounding), true, c.st);
+  if ((rc = check_workspace(ws_layout(M, N, 0), workspace, workspace_bytes))) return rc;
+  return run_rq_blocks<B_Q8_0>(rq_args(dense, packed_out, nullptr, nullptr, M, N, rounding), dense_dtype, is_sr(rounding),
+                               workspace, (hipStream_t)stream);
 }
 bool gguf_block_sizes(int type, int* bs, int* ts);                                       // lm_gguf.hip
 int gguf_dequant_run(const uint8_t* src, int type, int64_t nelem, void* out, int dt, hipStream_t st);  // lm_gguf.hip
@@ -78,5 +76,5 @@ extern "C" int lm_gguf_dequant(const uint8_t* packed, int32_t quant_type, int64_
   a.q = packed;
   a.out = out;
   a.out_dt = out_dtype;
-  return run_blocks<B_Q8_0, P_TODENSE>(a, lora->dtype, c.nkc, false, false, c.st);
+  return run_blocks<B_Q8_0, P_TODENSE>(a, lora->dtype, c.nkc, false, c.st);
 }

@@ -321,11 +321,11 @@ extern "C" int lm_nvfp4_merge_stack(const lm_stack_item* items, int32_t count, i
     const bool sr = rounding_mode == LM_ROUND_STOCHASTIC;
     if (swizzled && (rc = zero_swizzle_pad((uint8_t*)s.scale_out, s.M, s.N / 16, st))) break;
     if (two) {
-      if ((rc = run_blocks<B_NVFP4, P_AMAX>(a, s.lora.dtype, c.nkc, false, false, st))) break;
-      if ((rc = run_blocks<B_NVFP4, P_QUANT>(a, s.lora.dtype, c.nkc, sr, false, st))) break;
+      if ((rc = run_blocks<B_NVFP4, P_AMAX>(a, s.lora.dtype, c.nkc, false, st))) break;
+      if ((rc = run_blocks<B_NVFP4, P_QUANT>(a, s.lora.dtype, c.nkc, sr, st))) break;
       if (run_finalize<B_NVFP4>(a, s.lora.dtype, st)) rc = fail(LM_EHIP, "finalize launch failed");
     } else {
-      rc = run_blocks<B_NVFP4, P_FULL>(a, s.lora.dtype, c.nkc, sr, false, st);
+      rc = run_blocks<B_NVFP4, P_FULL>(a, s.lora.dtype, c.nkc, sr, st);
     }
   }
   free(preps);
