@@ -52,7 +52,8 @@ struct NvArgs {
 };
 struct NvStackItem {
   NvArgs a;
-  int64_t tile_begin;    // prefix of 32-row units (quant launches)
+  int64_t tile_begin;    // prefix of 32-row x column-chunk units (quant launches)
+  int chunks;            // column chunks per 32 rows (nv_chunks)
   int64_t bound_begin;   // prefix of 128-row chunks (pruned amax: bound launch)
   int64_t refine_begin;  // prefix of 512-tile chunks (pruned amax: refine launch)
 };
@@ -86,16 +87,15 @@ struct NvLane {
   uint32_t lsc_off;             // the lane's scale pair in the staged block (tile t0)
 };
 
-// Block scales staged in LDS (stacks in the plain layout whose rows have at
-// most NV_LSC_TILES macro tiles): the quant workgroup reads its 32 rows'
-// scale bytes of tiles [t0, t1) with 8-byte loads that cover whole lines,
-// each lane reads and writes its 2 bytes per tile in LDS, and the workgroup
-// writes the block back after its last tile.  Per tile and row group that
-// takes the 2-byte scale load and store off the texture-address unit, which
-// bounds round-to-nearest, and the partial-line scale traffic off HBM.  A
-// row's bytes sit NV_LSC_STRIDE apart: 8 * 129, so the 16 rows a load reads
-// fall in distinct banks.
-constexpr int NV_LSC_TILES = 128;
+// Block scales staged in LDS (stacks in the plain layout): the quant workgroup
+// reads its 32 rows' scale bytes of tiles [t0, t1) with 8-byte loads that
+// cover whole lines, each lane reads and writes its 2 bytes per tile in LDS,
+// and the workgroup writes the block back after its last tile.  Per tile and
+// row group that takes the 2-byte scale load and store off the
+// texture-address unit, which bounds round-to-nearest, and the partial-line
+// scale traffic off HBM.  A row's bytes sit NV_LSC_STRIDE apart: 8 * 33, so
+// the 16 rows a load reads fall in distinct banks.
+constexpr int NV_LSC_TILES = 4 * NV_NW;  // a column chunk (nv_chunks)
 constexpr int NV_LSC_STRIDE = 8 * (NV_LSC_TILES + 1);
 
 // row0: the 16-row group's first row (wave-uniform); rowc: the lane's row,
@@ -320,35 +320,34 @@ DEV void nv_quant_tile(const NvArgs& a, const NvTileIn<NKC>& in, const v4i16 (&b
 }
 
 // the staged block: rows row0 .. row0 + 31 (rows past M repeat row M - 1),
-// tiles [t0, t1), 8 bytes each; wave w moves rows w, w + 8, ...
+// tiles [t0, t1), 8 bytes each; a half wave moves one row
+static_assert(NV_LSC_TILES <= 32, "a half wave's lanes cover a chunk");
 DEV void nv_lsc_load(const NvArgs& a, int64_t row0, int t0, int t1, uint8_t* lsc) {
-  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int lane = threadIdx.x & 63, wave = wave_index(), c = lane & 31;
   const LM_GLOBAL uint8_t* sb = (const LM_GLOBAL uint8_t*)a.scale + 8 * t0;
   const int64_t scols = a.N >> 4;
 #pragma unroll
-  for (int i = 0; i < 32 / NV_NW; ++i) {
-    const int r = wave + NV_NW * i;
+  for (int i = 0; i < 32 / (2 * NV_NW); ++i) {
+    const int r = 2 * (wave + NV_NW * i) + (lane >> 5);
     const int64_t rr = row0 + r < a.M ? row0 + r : a.M - 1;
-    for (int c = lane; c < t1 - t0; c += 64)
-      *(lm_u32x2*)(lsc + r * NV_LSC_STRIDE + 8 * c) = *(const LM_GLOBAL lm_u32x2*)(sb + (rr * scols + 8 * c));
+    if (c < t1 - t0) *(lm_u32x2*)(lsc + r * NV_LSC_STRIDE + 8 * c) = *(const LM_GLOBAL lm_u32x2*)(sb + (rr * scols + 8 * c));
   }
 }
 DEV void nv_lsc_store(const NvArgs& a, int64_t row0, int t0, int t1, const uint8_t* lsc) {
-  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int lane = threadIdx.x & 63, wave = wave_index(), c = lane & 31;
   LM_GLOBAL uint8_t* sb = (LM_GLOBAL uint8_t*)a.scale_out + 8 * t0;
   const int64_t scols = a.N >> 4;
 #pragma unroll
-  for (int i = 0; i < 32 / NV_NW; ++i) {
-    const int r = wave + NV_NW * i;
-    if (row0 + r >= a.M) break;  // wave-uniform
-    for (int c = lane; c < t1 - t0; c += 64)
+  for (int i = 0; i < 32 / (2 * NV_NW); ++i) {
+    const int r = 2 * (wave + NV_NW * i) + (lane >> 5);
+    if (row0 + r < a.M && c < t1 - t0)
       *(LM_GLOBAL lm_u32x2*)(sb + ((row0 + r) * scols + 8 * c)) = *(const lm_u32x2*)(lsc + r * NV_LSC_STRIDE + 8 * c);
   }
 }
 
 // ---- pass bodies -------------------------------------------------------------
 // Rows past M load row M-1 (valid memory) and store nothing.
-// Tiles [t0, t1) of rows row0 .. row0+15 (the stack passes whole rows).
+// Tiles [t0, t1) of rows row0 .. row0+31.
 // the copy of the input per-tensor scale in red[1], which the quant pass reads
 DEV void nv_keep_gin(uint32_t* red, float gin) { ((LM_GLOBAL uint32_t*)red)[1] = f2u(gin); }
 
@@ -452,8 +451,17 @@ DEV int nv_find(const NvStackItem* __restrict__ items, int count, int64_t t) {
 }
 
 // ---- kernels: single tensor (args by value) and grouped (descriptor table) ---
-// One quant workgroup per 32 rows (tile_begin counts 32-row units).
-__host__ __device__ static inline int64_t nv_units(int64_t M, int64_t /*N*/) { return (M + 31) / 32; }
+// Stacks: one quant workgroup per 32 rows and column chunk.  A chunk has at
+// most 4 tiles per wave (32 tiles, a whole 4096-column row) and the row's
+// tiles are spread evenly over its chunks.  With whole rows a 14336-column unit took 3.5
+// times as long as a 4096-column one, and one 8B layer (1344 units for 512
+// resident workgroups, the long ones last) ended on them: 203 -> 123 us per
+// merge of a layer (round to nearest), 280 -> 151 (stochastic), 218 -> 139
+// (swizzled); 8 layers 677 -> 667 and 889 -> 872.  Only a swizzled stack of
+// many units is better off with whole rows (8 layers, stochastic: 917 us,
+// chunked 928): without staged scales a chunk saves nothing but the tail.
+__host__ __device__ static inline int nv_chunks(int64_t N) { return (int)(((N >> 7) + 4 * NV_NW - 1) / (4 * NV_NW)); }
+constexpr int64_t NV_WHOLE_ROWS = 8 * 512;  // 32-row units from which a swizzled stack keeps whole rows
 
 // Single tensors: blocks are independent once the global scale is known, so a
 // workgroup owns 32 rows x NV_CHUNK macro tiles (blockIdx.y picks the chunk).
@@ -478,8 +486,8 @@ __global__ __launch_bounds__(NV_NW * 64) void k_nv_quant(NvArgs a) {
                               TWO ? red[0] : 0u, TWO ? red[1] : 0u);
 }
 // TWO: every item of the launch is two-level (the host splits a mixed stack);
-// LSC: block scales staged in LDS, every item's rows have at most
-// NV_LSC_TILES macro tiles (the staging's barrier also covers rtab)
+// LSC: block scales staged in LDS (plain layout; the staging's barrier also
+// covers rtab)
 template <int NKC, bool SR, bool TWO, bool LSC>
 __global__ __launch_bounds__(NV_NW * 64) void k_nv_quant_stack(const NvStackItem* __restrict__ items, int count) {
   __shared__ float rtab[8];
@@ -489,8 +497,15 @@ __global__ __launch_bounds__(NV_NW * 64) void k_nv_quant_stack(const NvStackItem
   const int i = nv_find(items, count, t);
   const NvArgs& a = items[i].a;
   const LM_GLOBAL uint32_t* red = (const LM_GLOBAL uint32_t*)a.red;
-  nv_quant_body<NKC, TWO, SR, LSC>(a, (t - items[i].tile_begin) * 32, 0, (int)(a.N >> 7), rtab,
-                                   TWO ? red[0] : 0u, TWO ? red[1] : 0u);
+  // unit u of nrg row groups: chunk u / nrg (of the row's steps of NV_NW
+  // tiles), rows 32 (u % nrg); neighbouring units then share a chunk's A^T and,
+  // in the swizzled layout, lines of block scales
+  const uint32_t u = (uint32_t)(t - items[i].tile_begin), nc = (uint32_t)items[i].chunks;
+  const uint32_t nrg = (uint32_t)((a.M + 31) / 32), ch = u / nrg, rg = u - ch * nrg;
+  const uint32_t nt = (uint32_t)(a.N >> 7), steps = (nt + NV_NW - 1) / NV_NW;
+  const uint32_t t0 = ch * steps / nc * NV_NW, t1 = (ch + 1) * steps / nc * NV_NW;
+  nv_quant_body<NKC, TWO, SR, LSC>(a, (int64_t)rg * 32, (int)t0, (int)(t1 < nt ? t1 : nt), rtab, TWO ? red[0] : 0u,
+                                   TWO ? red[1] : 0u);
 }
 // ---- the pruned per-tensor amax (two-level) ---------------------------------
 // max |merged| over a tensor without merging every element.  For element
@@ -723,7 +738,7 @@ static inline bool nv_fast_ok(int cd, int nkc, int64_t M, int64_t N) {
 // single tensor: the pruned amax (two-level; prep gave it the factors' norms),
 // then quant on `st`
 static int nv_fast_run(const NvArgs& a, int nkc, bool sr, hipStream_t st) {
-  const dim3 grid((unsigned)nv_units(a.M, a.N), (unsigned)(((a.N >> 7) + NV_CHUNK - 1) / NV_CHUNK)), block(NV_NW * 64);
+  const dim3 grid((unsigned)((a.M + 31) / 32), (unsigned)(((a.N >> 7) + NV_CHUNK - 1) / NV_CHUNK)), block(NV_NW * 64);
   if (a.gin) {
     if (a.nrm == nullptr || a.ub == nullptr) return fail(LM_EINVAL, "nvfp4 two-level merge without its norm workspace");
     TimedLaunch timed("nvfp4", st);

@@ -184,6 +184,9 @@ static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swiz
   int64_t tiles[2] = {0, 0};
   int64_t bounds = 0, refines = 0;  // the pruned amax: 128-row bound chunks, 512-tile refine chunks
   int slot[2] = {0, n_two};
+  int64_t row_units = 0;
+  for (int i = 0; i < count; ++i) row_units += (items[i].M + 31) / 32;
+  const bool chunked = !swizzled || row_units < NV_WHOLE_ROWS;
   int rc = LM_OK;
   for (int i = 0; i < count && rc == LM_OK; ++i) {
     const lm_stack_item& s = items[i];
@@ -210,7 +213,8 @@ static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swiz
     a.swizzled = swizzled;
     a.seed = s.seed;
     it.tile_begin = tiles[grp];
-    tiles[grp] += nv_units(s.M, s.N);
+    it.chunks = chunked ? nv_chunks(s.N) : 1;
+    tiles[grp] += (s.M + 31) / 32 * it.chunks;
     it.bound_begin = bounds;
     it.refine_begin = refines;
     if (grp == 0) {
@@ -220,14 +224,12 @@ static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swiz
     if (rc == LM_OK && swizzled) rc = zero_swizzle_pad((uint8_t*)s.scale_out, s.M, s.N / 16, st);
   }
   if (rc == LM_OK) rc = lm_stage_h2d(dev_items, h, sizeof(NvStackItem) * count, st);
-  if (rc == LM_OK && (bounds > 0x7fffffff || refines > 0x7fffffff))
+  if (rc == LM_OK && (bounds > 0x7fffffff || refines > 0x7fffffff || tiles[0] > 0x7fffffff || tiles[1] > 0x7fffffff))
     rc = fail(LM_EUNSUPPORTED, "nvfp4 stack too large for one launch");
   const int nkc = preps[0].rpad / 16;
   const dim3 block(NV_NW * 64);
   const NvStackItem* d = (const NvStackItem*)dev_items;
-  // block scales staged in LDS: plain layout, rows of at most NV_LSC_TILES macro tiles
-  bool lsc = !swizzled;
-  for (int i = 0; i < count; ++i) lsc = lsc && (items[i].N >> 7) <= NV_LSC_TILES;
+  const bool lsc = !swizzled;  // plain block scales are staged in LDS
   if (rc == LM_OK && n_two > 0) {
     TimedLaunch timed("nvfp4", st);
     NKC_SWITCH(nkc_bucket(nkc), hipLaunchKernelGGL((k_nv_bound_stack<NKC_>), dim3((unsigned)bounds), block, 0, st, d,
