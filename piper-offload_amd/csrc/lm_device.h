@@ -99,6 +99,12 @@ DEV float row_max16(float x) {  // max over each 16-lane row
 }
 DEV float wave_max(float x) { return lanes_max32(lanes_max16(row_max16(x))); }
 
+// raise *slot (bits of a non-negative float) to v.  Most callers find it raised
+// already, and a load does not serialize as atomics on one line do.
+DEV void raise_max(uint32_t* slot, uint32_t v) {
+  if (v > __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(slot, v);
+}
+
 template <int DT>
 DEV float round_dt(float x) {
   if constexpr (DT == BF16) return bf16r(x);

@@ -2,6 +2,7 @@
 #include "lm_dequant.h"
 #include "lm_group.h"
 #include "lm_requant.h"
+#include "lm_tensor.h"
 
 // ---------------------------------------------------------------------------
 // FP8
@@ -26,7 +27,8 @@ static int fp8_merge(const uint8_t* q, const float* scale, uint8_t* q_out, float
   const bool split = group == N && rows_split_wanted(KIND, cd, LM_F32, false, sr, rpad_of(lora->rank) / 16, M, N);
   Ctx c;
   if ((rc = setup(c, M, N, lora, ws, wsb, stream, split))) return rc;
-  if (group == N || group != M * N) {  // per-row, or per-group
+  const bool tensor = group == M * N && group != N;
+  if (!tensor || tensor_fast_ok(KIND, cd, LM_F32, false, c.nkc, M, N)) {
     RowArgs a;
     memset(&a, 0, sizeof a);
     a.q = q;
@@ -39,7 +41,8 @@ static int fp8_merge(const uint8_t* q, const float* scale, uint8_t* q_out, float
     a.N = N;
     a.strength = lora->strength;
     a.seed = seed_of(rnd);
-    a.red = split ? c.red : nullptr;
+    a.red = split || tensor ? c.red : nullptr;
+    if (tensor) return tensor_merge_run(a, KIND, c.nkc, sr, c.st);
     if (group != N) return run_groups<KIND, false>(a, group, cd, LM_F32, false, sr, c.nkc, c.st);
     return run_rows<KIND, false>(a, cd, LM_F32, false, sr, c.nkc, c.st);
   }

@@ -1660,8 +1660,10 @@ __global__ __launch_bounds__(256) void k_blocks(BlkArgs a) {
     if (threadIdx.x == 0) {
       float x = __builtin_fmaxf(__builtin_fmaxf(sh_red[0][0], sh_red[0][1]), __builtin_fmaxf(sh_red[0][2], sh_red[0][3]));
       float y = __builtin_fmaxf(__builtin_fmaxf(sh_red[1][0], sh_red[1][1]), __builtin_fmaxf(sh_red[1][2], sh_red[1][3]));
-      atomicMax(&a.red[0], f2u(x));  // non-negative floats order like their bits
-      atomicMax(&a.red[1], f2u(y + 0.0f));
+      // non-negative floats order like their bits; a workgroup whose maximum
+      // another has reached skips the atomic (all of them share one line)
+      raise_max(&a.red[0], f2u(x));
+      raise_max(&a.red[1], f2u(y + 0.0f));
     }
   }
 }

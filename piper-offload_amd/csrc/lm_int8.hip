@@ -2,6 +2,7 @@
 #include "lm_dequant.h"
 #include "lm_group.h"
 #include "lm_requant.h"
+#include "lm_tensor.h"
 
 // ---------------------------------------------------------------------------
 // INT8
@@ -36,7 +37,8 @@ extern "C" int lm_int8_merge(const int8_t* q, const void* scale, const int8_t* z
   Ctx c;
   if ((rc = setup(c, M, N, lora, workspace, workspace_bytes, stream, split))) return rc;
   const int qmin = reduce_range ? -64 : -128, qmax = reduce_range ? 63 : 127;
-  if (group == N || group != M * N) {  // per-row, or per-group
+  const bool tensor = group == M * N && group != N;
+  if (!tensor || tensor_fast_ok(K_INT8, cd, scale_dtype, asym, c.nkc, M, N)) {
     RowArgs a;
     memset(&a, 0, sizeof a);
     a.q = q;
@@ -53,7 +55,8 @@ extern "C" int lm_int8_merge(const int8_t* q, const void* scale, const int8_t* z
     a.qmin = qmin;
     a.qmax = qmax;
     a.seed = seed_of(rounding);
-    a.red = split ? c.red : nullptr;
+    a.red = split || tensor ? c.red : nullptr;
+    if (tensor) return tensor_merge_run(a, K_INT8, c.nkc, sr, c.st);
     if (group != N) return run_groups<K_INT8, false>(a, group, cd, scale_dtype, asym, sr, c.nkc, c.st);
     return run_rows<K_INT8, false>(a, cd, scale_dtype, asym, sr, c.nkc, c.st);
   }

@@ -1,0 +1,17 @@
+// lm_tensor.h -- the fast per-tensor merges (lm_tensor.hip, a translation unit
+// of its own).
+#pragma once
+#include "lm_impl.h"
+
+// a.red: the workspace reduction slots that the prep launch cleared.  For the
+// layouts of tensor_fast_ok.
+__attribute__((visibility("hidden"))) int tensor_merge_run(const RowArgs& a, int kind, int nkc, bool sr, hipStream_t st);
+
+// The row kernels' 32-bit offsets and 64-column tiles, fp32 scales, symmetric
+// codes.  The amax pass has at most ceil(M / 64) ceil(N / 1024) workgroups,
+// whose partials take the 2 Mpad words that follow the first 64 reduction
+// slots: short weights of very long rows do not fit and run k_blocks.
+static inline bool tensor_fast_ok(int kind, int cd, int sdt, bool asym, int nkc, int64_t M, int64_t N) {
+  return sdt == LM_F32 && rows_fast_ok(kind, cd, sdt, asym, nkc, M, N) &&
+         (M + 63) / 64 * ((N + 1023) / 1024) <= red_words(M) - 64;
+}
