@@ -13,18 +13,16 @@
 //   out    = dt(y + total)
 //
 // At most 16 tokens (decode): one kernel, k_routed_small, and no workspace.
-// Otherwise three:
-// * k_routed_down: MFMA x A^T over a K split per workgroup; the partial sums
-//   of all factors' rank chunks go to an fp32 workspace [S][T][C * 16]
-//   (C = sum of ceil(r_i / 16));
-// * k_routed_finalize: sums the S partials in split order and writes
-//   ps = dt(dt(p) s) once per token, in the dtype, [T][C * 16];
+// Otherwise two:
+// * k_routed_down: MFMA x A^T, one 16-wave workgroup per 16 tokens whose waves
+//   split K and meet in LDS; writes ps = dt(dt(p) s) in the dtype, [T][C * 16]
+//   (C = sum of ceil(r_i / 16) rank chunks);
 // * k_routed_up: a wave keeps the B operands of one 64-column tile in
 //   registers and walks 16-token tiles: one MFMA chain per factor, the rest
 //   of the rounding chain and one read and one write of y / out: the only
 //   traffic that scales with T N.
 // Lane layout (the merge kernels' convention): a wave owns 16 tokens; lane l
-// holds token l & 15 and columns 16 (l >> 4) .. + 15 of a 64-column tile.
+// holds token l & 15 and 16 columns of a 64-column tile (up_col).
 #include "lm_impl.h"
 
 namespace {
@@ -37,11 +35,9 @@ struct RoutedArgs {
   const uint16_t* x;    // [T, K]
   const uint16_t* y;    // [T, N] (the Linear output)
   uint16_t* out;        // [T, N] (may alias y)
-  float* part;          // [S][T][C * 16]
   uint16_t* ps;         // [T][C * 16]: dt(dt(p) s) of each factor's ranks (zero past the rank)
   int64_t T, K, N;
-  int64_t kspan;        // K columns per split (multiple of 16)
-  int S, nf, nchunks;
+  int nf, nchunks;
   int tiles_per_wg;     // token tiles per up workgroup
   const uint16_t* a[RT_MAX_FACTORS];
   const uint16_t* b[RT_MAX_FACTORS];
@@ -107,83 +103,123 @@ __device__ __forceinline__ v4f32 mfma1(const v4i16& a, const v4i16& b, const v4f
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
 }
 
-// grid (token tiles, S); RT_NW waves split the workgroup's K range.  For rank
-// chunk c the MFMA computes D[r][t] = sum_k A_i[r][k] x[t][k]: lane l holds
-// ranks 16 c' + 4 (l >> 4) + 0..3 of token l & 15.  The waves' sums meet in
-// LDS, one chunk at a time, and wave 0 writes the split's partial.
-template <bool HALF>
-__global__ __launch_bounds__(RT_NW * 64) void k_routed_down(RoutedArgs a) {
-  __shared__ float sh[RT_NW][64][4];
+// grid (token tiles).  The workgroup's 16 waves split K: a round is RT_DU steps
+// of 32 columns per wave, in pairs of 64 neighbouring columns whose rows load as
+// whole cache lines (trade_rows8); all of a round's loads are issued before the
+// MFMAs (K = 4096 is one round).  For rank chunk c the MFMA computes
+// D[r][t] = sum_k A_i[r][k] x[t][k]: lane l holds ranks 16 c' + 4 (l >> 4) + 0..3
+// of token l & 15.  CB chunks share each round's x values; the waves' sums meet
+// in LDS and one thread per (chunk, rank, token) adds them in wave order and
+// rounds.  What bounds it is one trip to memory: with the K range split over
+// 2048 four-wave workgroups, fp32 partials and a kernel that summed them, 4096
+// tokens of K = 4096 took 11.3 + 4.8 us, and this takes 11.
+constexpr int RT_DNW = 16;
+constexpr int RT_DU = 8;
+// columns k .. k + 63 of rows row0 .. row0 + 15 as two accesses of whole lines;
+// trade_pair then gives lane (rl, g) columns k + 8 g .. and k + 32 + 8 g .. of row rl
+__device__ __forceinline__ void load_pair(const uint16_t* p, int64_t rows, int64_t cols, int64_t row0, int64_t k, int rl,
+                                          int g, rt_v8i16& v0, rt_v8i16& v1) {
+  const int64_t c = k + 32 * (rl >> 3) + 8 * g;
+  const rt_v8i16 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  v0 = c < cols ? load8(p, rows, cols, row0 + (rl & 7), c) : zero;
+  v1 = c < cols ? load8(p, rows, cols, row0 + (rl & 7) + 8, c) : zero;
+}
+__device__ __forceinline__ void trade_pair(rt_v8i16& v0, rt_v8i16& v1) {
+  lm_u32x4 x = __builtin_bit_cast(lm_u32x4, v0), y = __builtin_bit_cast(lm_u32x4, v1);
+  trade_rows8(x, y);
+  v0 = __builtin_bit_cast(rt_v8i16, x);
+  v1 = __builtin_bit_cast(rt_v8i16, y);
+}
+template <bool HALF, int CB>
+__global__ __launch_bounds__(RT_DNW * 64) void k_routed_down(RoutedArgs a) {
+  constexpr int DT = HALF ? F16 : BF16;
+  __shared__ float sh[CB][RT_DNW][256];
   const int lane = threadIdx.x & 63, wave = wave_index(), rl = lane & 15, g = lane >> 4;
   const int64_t t0 = (int64_t)blockIdx.x * 16;
-  const int split = blockIdx.y;
-  const int64_t kb = (int64_t)split * a.kspan, ke = kb + a.kspan < a.K ? kb + a.kspan : a.K;
-  for (int i = 0; i < a.nf; ++i) {
-    const int nck = (a.rank[i] + 15) / 16;
-    for (int cc = 0; cc < nck; ++cc) {
-      // RT_DU K steps of 32 per round: their 16-byte loads are all issued
-      // before the MFMAs (loads past K, the split or the rows read zeros)
-      constexpr int RT_DU = 8;
-      v4f32 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-      for (int64_t k0 = kb + 32 * wave; k0 < ke; k0 += 32 * RT_NW * RT_DU) {
-        rt_v8i16 av[RT_DU], xv[RT_DU];
+  for (int c0 = 0; c0 < a.nchunks; c0 += CB) {
+    v4f32 acc[CB];
 #pragma unroll
-        for (int u = 0; u < RT_DU; ++u) {
-          const int64_t k = k0 + (int64_t)u * 32 * RT_NW + 8 * g;
-          const bool in = k < ke;
-          av[u] = in ? load8(a.a[i], a.rank[i], a.K, 16 * cc + rl, k) : (rt_v8i16){0, 0, 0, 0, 0, 0, 0, 0};
-          xv[u] = in ? load8(a.x, a.T, a.K, t0 + rl, k) : (rt_v8i16){0, 0, 0, 0, 0, 0, 0, 0};
+    for (int c = 0; c < CB; ++c) acc[c] = (v4f32){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int64_t k0 = 64 * wave; k0 < a.K; k0 += 32 * RT_DNW * RT_DU) {
+      // loads past K or the rows read zeros
+      rt_v8i16 av[RT_DU], xv[RT_DU];
+#pragma unroll
+      for (int u = 0; u < RT_DU; u += 2) load_pair(a.x, a.T, a.K, t0, k0 + (int64_t)u * 32 * RT_DNW, rl, g, xv[u], xv[u + 1]);
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+        if (c0 + c >= a.nchunks) break;
+        const int i = a.cfac[c0 + c], cc = c0 + c - a.chunk0[i];
+#pragma unroll
+        for (int u = 0; u < RT_DU; u += 2)
+          load_pair(a.a[i], a.rank[i], a.K, 16 * cc, k0 + (int64_t)u * 32 * RT_DNW, rl, g, av[u], av[u + 1]);
+#pragma unroll
+        for (int u = 0; u < RT_DU; u += 2) {
+          trade_pair(av[u], av[u + 1]);
+          if (c == 0) trade_pair(xv[u], xv[u + 1]);
+          acc[c] = mfma32<HALF>(av[u], xv[u], acc[c]);
+          acc[c] = mfma32<HALF>(av[u + 1], xv[u + 1], acc[c]);
         }
-#pragma unroll
-        for (int u = 0; u < RT_DU; ++u) acc = mfma32<HALF>(av[u], xv[u], acc);
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sh[wave][lane][j] = acc[j];
-      __syncthreads();
-      const int64_t t = t0 + rl;
-      if (wave == 0 && t < a.T) {
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float sum = 0.0f;
-          for (int w = 0; w < RT_NW; ++w) sum += sh[w][lane][j];
-          v[j] = sum;
-        }
-        const int c = a.chunk0[i] + cc;
-        float* dst = a.part + ((int64_t)split * a.T + t) * (a.nchunks * 16) + c * 16 + 4 * g;
-        *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
-      }
-      __syncthreads();
     }
+#pragma unroll
+    for (int c = 0; c < CB; ++c) *(v4f32*)&sh[c][wave][4 * lane] = acc[c];
+    __syncthreads();
+    for (int o = threadIdx.x; o < CB * 256; o += RT_DNW * 64) {
+      const int c = o >> 8, e = o & 255;  // entry e: token (e >> 2) & 15, rank 4 (e >> 6) + (e & 3)
+      const int64_t t = t0 + ((e >> 2) & 15);
+      if (c0 + c < a.nchunks && t < a.T) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < RT_DNW; ++w) sum += sh[c][w][e];
+        a.ps[t * (a.nchunks * 16) + (c0 + c) * 16 + 4 * (e >> 6) + (e & 3)] =
+            bits_dt<DT>(round_dt<DT>(round_dt<DT>(sum) * a.s[a.cfac[c0 + c]]));
+      }
+    }
+    if (c0 + CB < a.nchunks) __syncthreads();  // the sums are read before the next chunks' overwrite them
   }
 }
 
-// one thread per (token, chunk, 4 ranks): sum the S partials in split order
-// and apply p_i = dt(p), ps_i = dt(p_i s_i)
-template <bool HALF>
-__global__ __launch_bounds__(256) void k_routed_finalize(RoutedArgs a) {
-  constexpr int DT = HALF ? F16 : BF16;
-  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (t, c, g)
-  const int64_t per_t = (int64_t)a.nchunks * 4;
-  if (q >= a.T * per_t) return;
-  const int64_t t = q / per_t;
-  const int rem = (int)(q - t * per_t), c = rem >> 2, g = rem & 3;
-  const int64_t off = t * (a.nchunks * 16) + c * 16 + 4 * g;
-  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int sp = 0; sp < a.S; ++sp) {
-    const float4 w = *(const float4*)(a.part + (int64_t)sp * a.T * (a.nchunks * 16) + off);
-    v[0] += w.x;
-    v[1] += w.y;
-    v[2] += w.z;
-    v[3] += w.w;
-  }
-  const float s_ = a.s[a.cfac[c]];
-  uint32_t w[2];
+// Columns of the up kernels: in a 64-column tile lane group g = lane >> 4 holds
+// columns 8 g .. 8 g + 7 (half 0, MFMAs 0 and 1) and 32 + 8 g .. + 7 (half 1,
+// MFMAs 2 and 3), so that one 16-byte access of the wave covers 64 contiguous
+// bytes of each of its 16 rows.  (With 16 consecutive columns per lane each
+// access touched every other 16 bytes: half of each sector per store.)
+__device__ __forceinline__ int up_col(int pos, int k4) {  // MFMA position -> column in the tile
+  return 32 * (k4 >> 1) + 8 * (pos >> 2) + 4 * (k4 & 1) + (pos & 3);
+}
+__device__ __forceinline__ int64_t up_col_of(int64_t mt, int g, int j) {  // the lane's value j, 0..15
+  return mt * 64 + 32 * (j >> 3) + 8 * g + (j & 7);
+}
+// y + total of one half (8 columns from c), rounded
+template <int DT>
+__device__ __forceinline__ lm_u32x4 up_sum8(const uint4& y, const float* total) {
+  const uint32_t yw[4] = {y.x, y.y, y.z, y.w};
+  uint32_t ow[4];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-    w[h] = (uint32_t)bits_dt<DT>(round_dt<DT>(round_dt<DT>(v[2 * h]) * s_)) |
-           ((uint32_t)bits_dt<DT>(round_dt<DT>(round_dt<DT>(v[2 * h + 1]) * s_)) << 16);
-  *(uint2*)(a.ps + off) = make_uint2(w[0], w[1]);
+  for (int k = 0; k < 4; ++k) {
+    const float lo = round_dt<DT>(val_dt<DT>(yw[k] & 0xffffu) + total[2 * k]);
+    const float hi = round_dt<DT>(val_dt<DT>(yw[k] >> 16) + total[2 * k + 1]);
+    ow[k] = (uint32_t)bits_dt<DT>(lo) | ((uint32_t)bits_dt<DT>(hi) << 16);
+  }
+  return lm_u32x4{ow[0], ow[1], ow[2], ow[3]};
+}
+// the lane's output of token t (vec: N % 8 == 0, halves are whole or outside)
+template <int DT>
+__device__ __forceinline__ void up_store(const RoutedArgs& a, int64_t t, int64_t mt, int g, bool vec, const uint4& y0,
+                                         const uint4& y1, const float (&total)[16]) {
+  uint16_t* orow = a.out + t * a.N;
+  const int64_t ca = mt * 64 + 8 * g, cb = ca + 32;
+  if (vec) {
+    if (ca < a.N) store_b128_guarded((LM_GLOBAL lm_u32x4*)(orow + ca), up_sum8<DT>(y0, total));
+    if (cb < a.N) store_b128_guarded((LM_GLOBAL lm_u32x4*)(orow + cb), up_sum8<DT>(y1, total + 8));
+  } else {
+    const uint16_t* yr = a.y + t * a.N;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int64_t c = up_col_of(mt, g, j);
+      if (c < a.N) orow[c] = bits_dt<DT>(round_dt<DT>(val_dt<DT>(yr[c]) + total[j]));
+    }
+  }
 }
 
 // grid (column-tile groups, token groups).  Every wave owns one 64-column
@@ -200,10 +236,10 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up(RoutedArgs a) {
   const int64_t mt = (int64_t)blockIdx.x * RT_NW + wave;  // the wave's column tile
   const int64_t ntiles = (a.N + 63) / 64;
   if (mt >= ntiles) return;
-  const int64_t c0 = mt * 64 + 16 * g;  // the lane's 16 output columns
-  const bool vec = (a.N & 7) == 0, full = vec && c0 + 16 <= a.N;
-  // B operands: MFMA k4, chunk c: position p = lane & 15 is column
-  // 16 (p >> 2) + 4 k4 + (p & 3), ranks 16 c' + 4 g + 0..3 of the chunk's factor
+  const int64_t ca = mt * 64 + 8 * g, cb = ca + 32;  // the lane's two runs of 8 output columns
+  const bool vec = (a.N & 7) == 0;
+  // B operands: MFMA k4, chunk c: position p = lane & 15 is column up_col(p, k4),
+  // ranks 16 c' + 4 g + 0..3 of the chunk's factor
   v4i16 bo[CMAX][4];
   const int p = lane & 15;
 #pragma unroll
@@ -212,7 +248,7 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up(RoutedArgs a) {
       const int i = a.cfac[c], cc = c - a.chunk0[i];
 #pragma unroll
       for (int k4 = 0; k4 < 4; ++k4)
-        bo[c][k4] = load4(a.b[i], a.N, a.rank[i], mt * 64 + 16 * (p >> 2) + 4 * k4 + (p & 3), 16 * cc + 4 * g);
+        bo[c][k4] = load4(a.b[i], a.N, a.rank[i], mt * 64 + up_col(p, k4), 16 * cc + 4 * g);
     }
   // bias * s of the lane's columns, per factor (rounded once)
   const int64_t tiles = (a.T + 15) / 16;
@@ -230,10 +266,10 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up(RoutedArgs a) {
       pv[c] = (v4i16){0, 0, 0, 0};
       if (c < a.nchunks && ok) pv[c] = __builtin_bit_cast(v4i16, *(const uint2*)(a.ps + t * rowstride + c * 16 + 4 * g));
     }
-    if (ok && full) {
-      const uint4* yr4 = (const uint4*)(a.y + t * a.N + c0);
-      v0 = yr4[0];
-      v1 = yr4[1];
+    if (ok && vec) {
+      const uint16_t* yr = a.y + t * a.N;
+      if (ca < a.N) v0 = *(const uint4*)(yr + ca);
+      if (cb < a.N) v1 = *(const uint4*)(yr + cb);
     }
   };
   load_tile(tb, pp, y0, y1);
@@ -261,30 +297,83 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up(RoutedArgs a) {
 #pragma unroll
           for (int j = 0; j < 16; ++j) {
             float part = round_dt<DT>(acc[j >> 2][j & 3]);
-            if (a.bias[i] && c0 + j < a.N)
-              part = round_dt<DT>(part + round_dt<DT>(val_dt<DT>(a.bias[i][c0 + j]) * a.s[i]));
+            if (a.bias[i] && up_col_of(mt, g, j) < a.N)
+              part = round_dt<DT>(part + round_dt<DT>(val_dt<DT>(a.bias[i][up_col_of(mt, g, j)]) * a.s[i]));
             total[j] = i == 0 ? part : round_dt<DT>(total[j] + part);
           }
         }
       }
     }
-    if (!tok || c0 >= a.N) continue;
-    uint16_t* orow = a.out + t * a.N + c0;
-    if (full) {
-      const uint32_t yw[8] = {cy0.x, cy0.y, cy0.z, cy0.w, cy1.x, cy1.y, cy1.z, cy1.w};
-      uint32_t ow[8];
+    if (tok) up_store<DT>(a, t, mt, g, vec, cy0, cy1, total);
+  }
+}
+
+// k_routed_up for one factor of rank <= 16 NC without a bias, N % 8 == 0: the
+// usual call, pared down to what it needs (62 VGPRs at rank 16, 8 waves per
+// SIMD).  y and out move in whole cache lines (trade_rows8), which is what bounds
+// it: 4096 tokens x 14336 took 53 us with 16 half lines per access and takes 42
+// now, near a copy's 41; deeper prefetch, wider workgroups and other orders of
+// the tiles changed nothing while the accesses were half lines.  A wave's
+// addresses are scalar bases that advance by a token tile plus constant 32-bit
+// lane offsets; the loads are unconditional (rows past T and columns past N
+// read valid ones), only the stores are predicated.
+template <bool HALF, int NC>
+__global__ __launch_bounds__(RT_NW * 64) void k_routed_up1(RoutedArgs a) {
+  constexpr int DT = HALF ? F16 : BF16;
+  const int lane = threadIdx.x & 63, wave = wave_index(), rl = lane & 15, g = lane >> 4;
+  const int64_t mt = (int64_t)blockIdx.x * RT_NW + wave;  // the wave's column tile
+  if (mt * 64 >= a.N) return;
+  const int N = (int)a.N, T = (int)a.T;
+  // the lane's piece of both accesses (trade_rows8): half rl >> 3 of row rl & 7 (+ 8)
+  const int col = (int)(mt * 64) + 32 * (rl >> 3) + 8 * g, r8 = rl & 7;
+  const bool cok = col < N;
+  v4i16 bo[NC][4];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float lo = round_dt<DT>(val_dt<DT>(yw[k] & 0xffffu) + total[2 * k]);
-        const float hi = round_dt<DT>(val_dt<DT>(yw[k] >> 16) + total[2 * k + 1]);
-        ow[k] = (uint32_t)bits_dt<DT>(lo) | ((uint32_t)bits_dt<DT>(hi) << 16);
-      }
-      ((uint4*)orow)[0] = make_uint4(ow[0], ow[1], ow[2], ow[3]);
-      ((uint4*)orow)[1] = make_uint4(ow[4], ow[5], ow[6], ow[7]);
-    } else {
-      const uint16_t* yr = a.y + t * a.N + c0;
-      for (int j = 0; j < 16 && c0 + j < a.N; ++j) orow[j] = bits_dt<DT>(round_dt<DT>(val_dt<DT>(yr[j]) + total[j]));
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int k4 = 0; k4 < 4; ++k4)
+      bo[c][k4] = load4(a.b[0], a.N, a.rank[0], mt * 64 + up_col(rl, k4), 16 * c + 4 * g);
+  const int tiles = (T + 15) >> 4;
+  const int tb = (int)blockIdx.y * a.tiles_per_wg, te = tb + a.tiles_per_wg < tiles ? tb + a.tiles_per_wg : tiles;
+  const uint32_t off0 = 2u * (uint32_t)(r8 * N + (cok ? col : 0)), off1 = off0 + 16u * (uint32_t)N;
+  const uint32_t offp = 2u * (uint32_t)(rl * (NC * 16) + 4 * g);
+  const uint32_t step = 32u * (uint32_t)N;  // bytes of a token tile
+  const LM_GLOBAL uint8_t* y = (const LM_GLOBAL uint8_t*)a.y;
+  const LM_GLOBAL uint8_t* ps = (const LM_GLOBAL uint8_t*)a.ps;
+  LM_GLOBAL uint8_t* out = (LM_GLOBAL uint8_t*)a.out;
+  lm_u32x4 y0, y1;
+  lm_u32x2 pv[NC];
+  auto load = [&](int tt) {
+    // a ragged last tile reads row T - 1 in place of the rows past it
+    const int last = T - 1 - 16 * tt;
+    const uint32_t b0 = r8 > last ? (uint32_t)(r8 - last) : 0u, b1 = r8 + 8 > last ? (uint32_t)(r8 + 8 - last) : 0u;
+    const uint32_t bp = rl > last ? (uint32_t)(rl - last) : 0u;
+    const LM_GLOBAL uint8_t* yt = y + (int64_t)tt * step;
+    y0 = *(const LM_GLOBAL lm_u32x4*)(yt + (off0 - b0 * 2u * (uint32_t)N));
+    y1 = *(const LM_GLOBAL lm_u32x4*)(yt + (off1 - b1 * 2u * (uint32_t)N));
+    const LM_GLOBAL uint8_t* pt = ps + (int64_t)tt * (NC * 512);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) pv[c] = *(const LM_GLOBAL lm_u32x2*)(pt + (offp - bp * (NC * 32u) + 32u * c));
+  };
+  load(tb);
+  for (int tt = tb; tt < te; ++tt) {
+    float total[16];
+#pragma unroll
+    for (int k4 = 0; k4 < 4; ++k4) {
+      v4f32 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc = mfma1<HALF>(bo[c][k4], __builtin_bit_cast(v4i16, pv[c]), acc);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) total[4 * k4 + j] = round_dt<DT>(acc[j]);
     }
+    trade_rows8(y0, y1);  // pieces a and b of the lane's own row
+    lm_u32x4 o0 = up_sum8<DT>(make_uint4(y0.x, y0.y, y0.z, y0.w), total);
+    lm_u32x4 o1 = up_sum8<DT>(make_uint4(y1.x, y1.y, y1.z, y1.w), total + 8);
+    load(tt + 1 < te ? tt + 1 : tt);
+    trade_rows8(o0, o1);
+    LM_GLOBAL uint8_t* ot = out + (int64_t)tt * step;
+    if (cok && 16 * tt + r8 < T) *(LM_GLOBAL lm_u32x4*)(ot + off0) = o0;
+    if (cok && 16 * tt + r8 + 8 < T) *(LM_GLOBAL lm_u32x4*)(ot + off1) = o1;
   }
 }
 
@@ -308,14 +397,14 @@ __global__ __launch_bounds__(RT_SNW * 64) void k_routed_small(RoutedArgs a) {
   const int lane = threadIdx.x & 63, wave = wave_index(), rl = lane & 15, g = lane >> 4;
   const int64_t mt = (int64_t)blockIdx.x * RT_SNW + wave;
   const bool tile = mt < (a.N + 63) / 64;
-  const int64_t c0 = mt * 64 + 16 * g, t = rl;
-  const bool tok = tile && t < a.T, full = (a.N & 7) == 0 && c0 + 16 <= a.N;
+  const int64_t ca = mt * 64 + 8 * g, cb = ca + 32, t = rl;
+  const bool tok = tile && t < a.T, vec = (a.N & 7) == 0;
   const int p = lane & 15;
   uint4 y0 = make_uint4(0, 0, 0, 0), y1 = y0;
-  if (tok && full) {
-    const uint4* yr4 = (const uint4*)(a.y + t * a.N + c0);
-    y0 = yr4[0];
-    y1 = yr4[1];
+  if (tok && vec) {
+    const uint16_t* yr = a.y + t * a.N;
+    if (ca < a.N) y0 = *(const uint4*)(yr + ca);
+    if (cb < a.N) y1 = *(const uint4*)(yr + cb);
   }
   v4i16 bo[PRE ? CMAX : 1][4];
   if constexpr (PRE) {
@@ -327,11 +416,10 @@ __global__ __launch_bounds__(RT_SNW * 64) void k_routed_small(RoutedArgs a) {
         const int i = a.cfac[c], cc = c - a.chunk0[i];
 #pragma unroll
         for (int k4 = 0; k4 < 4; ++k4)
-          bo[c][k4] = load4(a.b[i], a.N, a.rank[i], mt * 64 + 16 * (p >> 2) + 4 * k4 + (p & 3), 16 * cc + 4 * g);
+          bo[c][k4] = load4(a.b[i], a.N, a.rank[i], mt * 64 + up_col(p, k4), 16 * cc + 4 * g);
       }
     }
   }
-  constexpr int RT_DU = 8;
   for (int c = 0; c < a.nchunks; ++c) {
     const int i = a.cfac[c], cc = c - a.chunk0[i];
     v4f32 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -386,58 +474,31 @@ __global__ __launch_bounds__(RT_SNW * 64) void k_routed_small(RoutedArgs a) {
         if constexpr (PRE)
           bv = bo[c][k4];
         else
-          bv = load4(a.b[i], a.N, a.rank[i], mt * 64 + 16 * (p >> 2) + 4 * k4 + (p & 3), 16 * cc + 4 * g);
+          bv = load4(a.b[i], a.N, a.rank[i], mt * 64 + up_col(p, k4), 16 * cc + 4 * g);
         acc[k4] = mfma1<HALF>(bv, psv, acc[k4]);
       }
       if (c + 1 == a.nchunks || a.cfac[c + 1] != i) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           float part = round_dt<DT>(acc[j >> 2][j & 3]);
-          if (a.bias[i] && c0 + j < a.N)
-            part = round_dt<DT>(part + round_dt<DT>(val_dt<DT>(a.bias[i][c0 + j]) * a.s[i]));
+          if (a.bias[i] && up_col_of(mt, g, j) < a.N)
+            part = round_dt<DT>(part + round_dt<DT>(val_dt<DT>(a.bias[i][up_col_of(mt, g, j)]) * a.s[i]));
           total[j] = i == 0 ? part : round_dt<DT>(total[j] + part);
         }
       }
     }
   }
-  if (!tok || c0 >= a.N) return;
-  uint16_t* orow = a.out + t * a.N + c0;
-  if (full) {
-    const uint32_t yw[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
-    uint32_t ow[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const float lo = round_dt<DT>(val_dt<DT>(yw[k] & 0xffffu) + total[2 * k]);
-      const float hi = round_dt<DT>(val_dt<DT>(yw[k] >> 16) + total[2 * k + 1]);
-      ow[k] = (uint32_t)bits_dt<DT>(lo) | ((uint32_t)bits_dt<DT>(hi) << 16);
-    }
-    ((uint4*)orow)[0] = make_uint4(ow[0], ow[1], ow[2], ow[3]);
-    ((uint4*)orow)[1] = make_uint4(ow[4], ow[5], ow[6], ow[7]);
-  } else {
-    const uint16_t* yr = a.y + t * a.N + c0;
-    for (int j = 0; j < 16 && c0 + j < a.N; ++j) orow[j] = bits_dt<DT>(round_dt<DT>(val_dt<DT>(yr[j]) + total[j]));
-  }
-}
-
-// K splits of the down projection: about 2048 workgroups in all (the kernel
-// streams x, so it needs occupancy), at least 256 columns of K per split
-int64_t routed_splits(int64_t T, int64_t K) {
-  const int64_t tiles = (T + 15) / 16;
-  int64_t S = (K + 255) / 256;
-  const int64_t want = (2048 + tiles - 1) / (tiles > 0 ? tiles : 1);
-  if (S > want) S = want;
-  return S < 1 ? 1 : S;
+  if (tok) up_store<DT>(a, t, mt, g, vec, y0, y1, total);
 }
 
 }  // namespace
 
 extern "C" size_t lm_routed_workspace_size(int64_t T, int64_t K, const lm_routed_factor* factors, int32_t count) {
   if (T <= 16) return 0;  // the single-launch path keeps everything in LDS
+  (void)K;
   int chunks = 0;
   for (int i = 0; i < count && factors; ++i) chunks += (factors[i].rank + 15) / 16;
-  const int64_t S = routed_splits(T, K);
-  const size_t tt = (size_t)(T > 0 ? T : 0) * (size_t)chunks * 16;
-  return align256((size_t)S * tt * sizeof(float)) + align256(tt * sizeof(uint16_t)) + 256;
+  return align256((size_t)T * (size_t)chunks * 16 * sizeof(uint16_t));  // ps
 }
 
 extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64_t T, int64_t K, int64_t N,
@@ -478,29 +539,26 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
     return fail(LM_EWORKSPACE, "routed residual workspace too small: %zu < %zu bytes", workspace_bytes, need);
   if (((uintptr_t)workspace & 255) != 0) return fail(LM_EINVAL, "workspace must be 256-byte aligned");
   const int64_t tiles = (T + 15) / 16;
-  const int64_t S = routed_splits(T, K);
   a.x = (const uint16_t*)x;
   a.y = (const uint16_t*)y;
   a.out = (uint16_t*)out;
-  a.part = (float*)workspace;
-  a.ps = (uint16_t*)((uint8_t*)workspace + align256((size_t)S * (size_t)T * (size_t)chunks * 16 * sizeof(float)));
+  a.ps = (uint16_t*)workspace;
   a.T = T;
   a.K = K;
   a.N = N;
-  a.S = (int)S;
-  a.kspan = ((K + S - 1) / S + 15) / 16 * 16;
   a.nf = count;
   a.nchunks = chunks;
   // up kernel: one 64-column tile per wave, token tiles split into groups so
-  // that there are about 4096 waves in all
+  // that there are about 8192 waves in all (4096 and 16384: 57.5 and 57.7
+  // against 56.3 us for 4096 tokens, 4096 -> 14336, rank 16)
   const int64_t ntiles = (N + 63) / 64;
   const int64_t colgroups = (ntiles + RT_NW - 1) / RT_NW;
-  int64_t tgroups = (4096 + ntiles - 1) / ntiles;
+  int64_t tgroups = (8192 + ntiles - 1) / ntiles;
   if (tgroups > tiles) tgroups = tiles;
   if (tgroups < 1) tgroups = 1;
   a.tiles_per_wg = (int)((tiles + tgroups - 1) / tgroups);
   tgroups = (tiles + a.tiles_per_wg - 1) / a.tiles_per_wg;
-  if (tiles > 0x7fffffff || S > 65535 || tgroups > 65535 || colgroups > 0x7fffffff)
+  if (tiles > 0x7fffffff || tgroups > 65535 || colgroups > 0x7fffffff)
     return fail(LM_EUNSUPPORTED, "routed residual grid too large");
   hipStream_t st = (hipStream_t)stream;
   TimedLaunch timed("routed", st);
@@ -518,21 +576,30 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
     return LM_OK;
   }
   const dim3 ugrid((unsigned)colgroups, (unsigned)tgroups);
+  // (32-bit lane offsets of a token tile)
+  const bool lean = count == 1 && !a.bias[0] && (N & 7) == 0 && chunks <= 4 && chunks != 3 && N < (INT64_C(1) << 26) &&
+                    T < (INT64_C(1) << 31) - 16;
 #define RT_UP(H_)                                                                                    \
-  if (chunks <= 1) hipLaunchKernelGGL((k_routed_up<H_, 1>), ugrid, block, 0, st, a);                \
+  if (lean && chunks == 1) hipLaunchKernelGGL((k_routed_up1<H_, 1>), ugrid, block, 0, st, a);        \
+  else if (lean && chunks == 2) hipLaunchKernelGGL((k_routed_up1<H_, 2>), ugrid, block, 0, st, a);   \
+  else if (lean) hipLaunchKernelGGL((k_routed_up1<H_, 4>), ugrid, block, 0, st, a);                  \
+  else if (chunks <= 1) hipLaunchKernelGGL((k_routed_up<H_, 1>), ugrid, block, 0, st, a);                \
   else if (chunks <= 2) hipLaunchKernelGGL((k_routed_up<H_, 2>), ugrid, block, 0, st, a);           \
   else if (chunks <= 4) hipLaunchKernelGGL((k_routed_up<H_, 4>), ugrid, block, 0, st, a);           \
   else hipLaunchKernelGGL((k_routed_up<H_, RT_MAX_CHUNKS>), ugrid, block, 0, st, a);
-  const dim3 fgrid((unsigned)((T * chunks * 4 + 255) / 256));
+#define RT_DOWN(H_)                                                                            \
+  if (chunks <= 1) hipLaunchKernelGGL((k_routed_down<H_, 1>), dgrid, dblock, 0, st, a);        \
+  else if (chunks <= 2) hipLaunchKernelGGL((k_routed_down<H_, 2>), dgrid, dblock, 0, st, a);   \
+  else hipLaunchKernelGGL((k_routed_down<H_, 4>), dgrid, dblock, 0, st, a);
+  const dim3 dgrid((unsigned)tiles), dblock(RT_DNW * 64);
   if (dtype == LM_F16) {
-    hipLaunchKernelGGL(k_routed_down<true>, dim3((unsigned)tiles, (unsigned)S), block, 0, st, a);
-    hipLaunchKernelGGL(k_routed_finalize<true>, fgrid, dim3(256), 0, st, a);
+    RT_DOWN(true)
     RT_UP(true)
   } else {
-    hipLaunchKernelGGL(k_routed_down<false>, dim3((unsigned)tiles, (unsigned)S), block, 0, st, a);
-    hipLaunchKernelGGL(k_routed_finalize<false>, fgrid, dim3(256), 0, st, a);
+    RT_DOWN(false)
     RT_UP(false)
   }
+#undef RT_DOWN
 #undef RT_UP
   LAUNCH_CHECK();
   return LM_OK;
