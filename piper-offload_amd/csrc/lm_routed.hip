@@ -498,7 +498,10 @@ extern "C" size_t lm_routed_workspace_size(int64_t T, int64_t K, const lm_routed
   (void)K;
   int chunks = 0;
   for (int i = 0; i < count && factors; ++i) chunks += (factors[i].rank + 15) / 16;
-  return align256((size_t)T * (size_t)chunks * 16 * sizeof(uint16_t));  // ps
+  // ps in the dtype, and room for p in fp32: the size that this entry point has
+  // promised callers since p was summed over launches
+  const size_t tt = (size_t)T * (size_t)chunks * 16;
+  return align256(tt * sizeof(float)) + align256(tt * sizeof(uint16_t));
 }
 
 extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64_t T, int64_t K, int64_t N,
