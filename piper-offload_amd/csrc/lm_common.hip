@@ -98,7 +98,7 @@ int launch_prep(const PrepItem& it, hipStream_t st) {
 
 
 // ---- host -> device staging of descriptor tables ---------------------------
-// The stack entries upload per-call descriptor tables.  They go through a
+// The stack entries upload per-call descriptor tables.  Large ones go through a
 // small pool of pinned host buffers, each guarded by an event recorded after
 // its copy, so the entry points return without synchronizing the stream: a
 // buffer is reused once its previous copy has completed (waiting on the
@@ -117,8 +117,37 @@ uint64_t g_stage_clock = 0;
 constexpr size_t kStageSlots = 8;
 }  // namespace
 
+// Small tables travel as kernel arguments (kUploadBytes per launch): a copy
+// between two kernels of a stream, through whatever engine, costs about 15 us
+// of idle GPU around its 4 us, a launch about 2 us and no staging slot.  Up to
+// kUploadLaunches of them; a larger table is one copy.
+namespace {
+constexpr size_t kUploadBytes = 3584;  // kernel arguments end at 4 KiB
+constexpr size_t kUploadLaunches = 4;
+struct UploadChunk {
+  uint32_t w[kUploadBytes / 4];
+};
+__global__ __launch_bounds__(256) void k_upload(UploadChunk c, uint32_t* dst, int words) {
+  for (int i = threadIdx.x; i < words; i += 256) ((LM_GLOBAL uint32_t*)dst)[i] = c.w[i];
+}
+}  // namespace
+
+// dst 4-byte aligned; whole words are written (the tables' regions are padded)
+static int upload_args(uint8_t* dst, const uint8_t* src, size_t bytes, hipStream_t st) {
+  for (size_t off = 0; off < bytes; off += kUploadBytes) {
+    const size_t n = bytes - off < kUploadBytes ? bytes - off : kUploadBytes;
+    UploadChunk c;
+    memcpy(c.w, src + off, n);
+    if (n % 4) memset((uint8_t*)c.w + n, 0, 4 - n % 4);
+    hipLaunchKernelGGL(k_upload, dim3(1), dim3(256), 0, st, c, (uint32_t*)(dst + off), (int)((n + 3) / 4));
+    LAUNCH_CHECK();
+  }
+  return LM_OK;
+}
+
 int lm_stage_h2d(void* dst, const void* src, size_t bytes, hipStream_t st) {
   if (bytes == 0) return LM_OK;
+  if (bytes <= kUploadBytes * kUploadLaunches) return upload_args((uint8_t*)dst, (const uint8_t*)src, bytes, st);
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(g_stage_mu);

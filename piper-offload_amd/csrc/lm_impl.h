@@ -273,7 +273,7 @@ static __global__ __launch_bounds__(256) void k_prep_many(const PrepItem* __rest
 }
 
 int launch_prep(const PrepItem& it, hipStream_t st);
-// asynchronous host -> device copy through pinned staging (lm_common.hip)
+// asynchronous host -> device copy of a descriptor table (lm_common.hip)
 int lm_stage_h2d(void* dst, const void* src, size_t bytes, hipStream_t st);
 
 // kernel timer (lm_timer_enable / lm_timer_read): bracket a launch on `st`

@@ -42,16 +42,18 @@ static int stack_layout(const lm_stack_item* items, int32_t count, void* ws, siz
   return LM_OK;
 }
 
-static int stack_prep(PrepItem* preps, int32_t count, uint8_t* dev_items, hipStream_t st) {
-  int64_t blocks = 0;
+// numbers the items' prep workgroups; the launch follows the table's upload
+static int stack_prep_blocks(PrepItem* preps, int32_t count, int64_t& blocks) {
+  blocks = 0;
   for (int i = 0; i < count; ++i) {
     preps[i].work_begin = 0;
     preps[i].block_begin = blocks;
     blocks += (prep_units(preps[i]) + PREP_PER_BLOCK - 1) / PREP_PER_BLOCK;
   }
   if (blocks > 0x7fffffff) return fail(LM_EUNSUPPORTED, "stack factors too large for one prep launch");
-  int rc = lm_stage_h2d(dev_items, preps, sizeof(PrepItem) * count, st);
-  if (rc != LM_OK) return rc;
+  return LM_OK;
+}
+static int stack_prep_launch(const uint8_t* dev_items, int32_t count, int64_t blocks, hipStream_t st) {
   TimedLaunch timed("prep", st);
   hipLaunchKernelGGL(k_prep_many, dim3((unsigned)blocks), dim3(256), 0, st, (const PrepItem*)dev_items, count);
   LAUNCH_CHECK();
@@ -68,23 +70,21 @@ extern "C" int lm_int8_merge_stack(const lm_stack_item* items, int32_t count, in
   const size_t extra = lm_stack_workspace_extra(count);
   if (workspace_bytes < extra) return fail(LM_EWORKSPACE, "stack workspace too small");
   uint8_t* base = (uint8_t*)workspace;
-  uint8_t* dev_prep = base;
   uint8_t* dev_rows = base + align256((size_t)count * sizeof(PrepItem));
   size_t cursor = extra;
-  // host tables; lm_stage_h2d copies them into pinned staging before returning
-  // the rows table and, right after its region, the items' first groups
-  // (begins, int32, in launch order): one upload into the RowStackItem and
-  // BlkArgs regions of the workspace (the INT8 stack does not use the latter)
+  // One host table in the layout of the workspace's descriptor regions, uploaded
+  // at once: the prep items, the row items and, right after their region, the
+  // items' first groups (begins, int32, in launch order; the BlkArgs region,
+  // which the INT8 stack does not use otherwise)
+  const size_t prep_bytes = align256((size_t)count * sizeof(PrepItem));
   const size_t rows_bytes = align256((size_t)count * sizeof(RowStackItem));
+  const size_t table_bytes = prep_bytes + rows_bytes + (size_t)count * sizeof(int32_t);
   static_assert(sizeof(BlkArgs) >= sizeof(int32_t), "begins fit the BlkArgs region");
-  PrepItem* preps = (PrepItem*)calloc(count, sizeof(PrepItem));
-  RowStackItem* rows = (RowStackItem*)calloc(1, rows_bytes + (size_t)count * sizeof(int32_t));
-  if (!preps || !rows) {
-    free(preps);
-    free(rows);
-    return fail(LM_EINVAL, "host allocation failed");
-  }
-  int32_t* begins = (int32_t*)((uint8_t*)rows + rows_bytes);
+  uint8_t* table = (uint8_t*)calloc(1, table_bytes);
+  if (!table) return fail(LM_EINVAL, "host allocation failed");
+  PrepItem* preps = (PrepItem*)table;
+  RowStackItem* rows = (RowStackItem*)(table + prep_bytes);
+  int32_t* begins = (int32_t*)(table + prep_bytes + rows_bytes);
   int rc = stack_layout(items, count, workspace, workspace_bytes, preps, cursor);
   int nkc_max = 0, cd = items[0].lora.dtype;
   for (int i = 0; i < count; ++i) {
@@ -131,7 +131,8 @@ extern "C" int lm_int8_merge_stack(const lm_stack_item* items, int32_t count, in
   }
   if (rc == LM_OK && (tiles[0] > 0x7fffffff || tiles[1] > 0x7fffffff))
     rc = fail(LM_EUNSUPPORTED, "stack too large for one launch");
-  if (rc == LM_OK) rc = stack_prep(preps, count, dev_prep, st);
+  int64_t prep_blocks = 0;
+  if (rc == LM_OK) rc = stack_prep_blocks(preps, count, prep_blocks);
   if (rc == LM_OK) {
     // every item uses the largest rank bucket: the prepared layouts are per item,
     // so items with a smaller rank must have the same padding.  Re-check.
@@ -139,7 +140,8 @@ extern "C" int lm_int8_merge_stack(const lm_stack_item* items, int32_t count, in
       if (nkc_bucket(rpad_of(items[i].lora.rank) / 16) != nkc_bucket(nkc_max))
         rc = fail(LM_EUNSUPPORTED, "stack items must share one rank bucket (16/32/64)");
   }
-  if (rc == LM_OK) rc = lm_stage_h2d(dev_rows, rows, rows_bytes + sizeof(int32_t) * count, st);
+  if (rc == LM_OK) rc = lm_stage_h2d(base, table, table_bytes, st);
+  if (rc == LM_OK) rc = stack_prep_launch(base, count, prep_blocks, st);
   const int32_t* dev_begins = (const int32_t*)(dev_rows + rows_bytes);
   if (rc == LM_OK) {
     const dim3 block(ROW_NW * 64);
@@ -163,20 +165,22 @@ extern "C" int lm_int8_merge_stack(const lm_stack_item* items, int32_t count, in
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(LM_EHIP, "stack launch: %s", hipGetErrorString(e));
   }
-  free(preps);
-  free(rows);
+  free(table);
   return rc;
 }
 
 // Grouped NVFP4 merge.  Two-level items: the pruned amax (bound-and-seed and
 // refine launches over all of them), then one quant launch; single-level
-// items: one quant launch.  `dev_items` is workspace for the descriptor table
-// (the BlkArgs region of lm_stack_workspace_extra).
-static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swizzled, bool sr, const PrepItem* preps,
-                         uint8_t* dev_items, hipStream_t st) {
+// items: one quant launch.  `table` is the host table, the prep items and then
+// the (still empty) NvStackItems, in the layout of the workspace `base`, whose
+// descriptor regions take it in one upload; `prep_blocks` workgroups of prep
+// follow it.
+static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swizzled, bool sr, uint8_t* table,
+                         uint8_t* base, int64_t prep_blocks, hipStream_t st) {
   static_assert(sizeof(NvStackItem) <= sizeof(BlkArgs), "NVFP4 stack descriptors must fit the workspace slot");
-  NvStackItem* h = (NvStackItem*)calloc(count, sizeof(NvStackItem));
-  if (!h) return fail(LM_EINVAL, "host allocation failed");
+  const PrepItem* preps = (const PrepItem*)table;
+  const size_t prep_bytes = align256((size_t)count * sizeof(PrepItem));
+  NvStackItem* h = (NvStackItem*)(table + prep_bytes);
   // two-level items first, then single-level ones; each group numbers its
   // 16-row units from 0 and gets its own quant launch
   int n_two = 0;
@@ -223,12 +227,13 @@ static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swiz
     }
     if (rc == LM_OK && swizzled) rc = zero_swizzle_pad((uint8_t*)s.scale_out, s.M, s.N / 16, st);
   }
-  if (rc == LM_OK) rc = lm_stage_h2d(dev_items, h, sizeof(NvStackItem) * count, st);
   if (rc == LM_OK && (bounds > 0x7fffffff || refines > 0x7fffffff || tiles[0] > 0x7fffffff || tiles[1] > 0x7fffffff))
     rc = fail(LM_EUNSUPPORTED, "nvfp4 stack too large for one launch");
+  if (rc == LM_OK) rc = lm_stage_h2d(base, table, prep_bytes + sizeof(NvStackItem) * count, st);
+  if (rc == LM_OK) rc = stack_prep_launch(base, count, prep_blocks, st);
   const int nkc = preps[0].rpad / 16;
   const dim3 block(NV_NW * 64);
-  const NvStackItem* d = (const NvStackItem*)dev_items;
+  const NvStackItem* d = (const NvStackItem*)(base + prep_bytes);
   const bool lsc = !swizzled;  // plain block scales are staged in LDS
   if (rc == LM_OK && n_two > 0) {
     TimedLaunch timed("nvfp4", st);
@@ -261,7 +266,6 @@ static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swiz
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(LM_EHIP, "nvfp4 quant launch: %s", hipGetErrorString(e));
   }
-  free(h);
   return rc;
 }
 
@@ -278,8 +282,10 @@ extern "C" int lm_nvfp4_merge_stack(const lm_stack_item* items, int32_t count, i
   if (workspace_bytes < extra) return fail(LM_EWORKSPACE, "stack workspace too small");
   uint8_t* base = (uint8_t*)workspace;
   size_t cursor = extra;
-  PrepItem* preps = (PrepItem*)calloc(count, sizeof(PrepItem));
-  if (!preps) return fail(LM_EINVAL, "host allocation failed");
+  const size_t prep_bytes = align256((size_t)count * sizeof(PrepItem));
+  uint8_t* table = (uint8_t*)calloc(1, prep_bytes + (size_t)count * sizeof(NvStackItem));
+  if (!table) return fail(LM_EINVAL, "host allocation failed");
+  PrepItem* preps = (PrepItem*)table;
   int rc = stack_layout(items, count, workspace, workspace_bytes, preps, cursor);
   bool fast = rc == LM_OK;
   for (int i = 0; fast && i < count; ++i)
@@ -291,13 +297,15 @@ extern "C" int lm_nvfp4_merge_stack(const lm_stack_item* items, int32_t count, i
     preps[i].norms = items[i].aux && items[i].lora.dtype == LM_BF16 ? 1 : 0;
     preps[i].at_order = fast && nkc_bucket(preps[0].rpad / 16) == 1 ? AT_NV16 : AT_PLAIN;
   }
-  if (rc == LM_OK) rc = stack_prep(preps, count, base, st);
+  int64_t prep_blocks = 0;
+  if (rc == LM_OK) rc = stack_prep_blocks(preps, count, prep_blocks);
   if (fast && rc == LM_OK) {
-    uint8_t* dev_blk = base + align256((size_t)count * sizeof(PrepItem)) + align256((size_t)count * sizeof(RowStackItem));
-    rc = nv_stack_fast(items, count, swizzled, rounding_mode == LM_ROUND_STOCHASTIC, preps, dev_blk, st);
-    free(preps);
+    rc = nv_stack_fast(items, count, swizzled, rounding_mode == LM_ROUND_STOCHASTIC, table, base, prep_blocks, st);
+    free(table);
     return rc;
   }
+  if (rc == LM_OK) rc = lm_stage_h2d(base, table, sizeof(PrepItem) * count, st);
+  if (rc == LM_OK) rc = stack_prep_launch(base, count, prep_blocks, st);
   lm_rounding rnd;
   rnd.mode = rounding_mode;
   rnd.reserved = 0;
@@ -330,6 +338,6 @@ extern "C" int lm_nvfp4_merge_stack(const lm_stack_item* items, int32_t count, i
       rc = run_blocks<B_NVFP4, P_FULL>(a, s.lora.dtype, c.nkc, sr, st);
     }
   }
-  free(preps);
+  free(table);
   return rc;
 }
