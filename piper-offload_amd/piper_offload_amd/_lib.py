@@ -7,6 +7,7 @@ There is no fallback: when the HIP library is missing or no GPU is present,
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -107,6 +108,8 @@ def library_path() -> str:
 def load_library() -> ctypes.CDLL:
     """Load the shared library and bind every exported signature (no GPU needed)."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not os.path.exists(_LIB_PATH):
@@ -126,7 +129,7 @@ def load_library() -> ctypes.CDLL:
 def lib() -> ctypes.CDLL:
     """Return the bound library for a GPU call; raises without a HIP device."""
     handle = load_library()
-    if not torch.cuda.is_available():
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():  # (is_available alone takes 2 us a call)
         raise RuntimeError("piper_offload_amd: the LoRA-merge kernels need a ROCm GPU (torch.cuda is unavailable)")
     return handle
 
@@ -158,18 +161,21 @@ def check(rc: int) -> None:
     raise RuntimeError(msg)
 
 
+_DTYPE_IDS = {torch.bfloat16: LM_BF16, torch.float16: LM_F16, torch.float32: LM_F32,
+              torch.float8_e4m3fn: LM_E4M3, torch.float8_e5m2: LM_E5M2}
+
+
 def torch_dtype_id(dtype: torch.dtype) -> int:
-    if dtype is torch.bfloat16:
-        return LM_BF16
-    if dtype is torch.float16:
-        return LM_F16
-    if dtype is torch.float32:
-        return LM_F32
-    if dtype is torch.float8_e4m3fn:
-        return LM_E4M3
-    if dtype is torch.float8_e5m2:
-        return LM_E5M2
-    raise ValueError(f"unsupported dtype {dtype}")
+    dtype_id = _DTYPE_IDS.get(dtype)
+    if dtype_id is None:
+        raise ValueError(f"unsupported dtype {dtype}")
+    return dtype_id
+
+
+@functools.lru_cache(maxsize=1024)
+def workspace_size(rows: int, cols: int, rank: int) -> int:
+    """``lm_workspace_size``, a function of the three numbers alone."""
+    return load_library().lm_workspace_size(rows, cols, rank)
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
@@ -196,5 +202,26 @@ def rounding_struct(rounding_seed: int | None) -> RoundingStruct:
     return RoundingStruct(LM_ROUND_STOCHASTIC, 0, int(rounding_seed))
 
 
+class on_device:
+    """``torch.cuda.device`` that does nothing when ``device`` is the current one already."""
+
+    __slots__ = ("index", "previous")
+
+    def __init__(self, device: torch.device) -> None:
+        self.index = device.index
+        self.previous = -1
+
+    def __enter__(self) -> None:
+        current = torch.cuda.current_device()
+        if self.index is not None and self.index != current:
+            torch.cuda.set_device(self.index)
+            self.previous = current
+
+    def __exit__(self, *exc: object) -> None:
+        if self.previous >= 0:
+            torch.cuda.set_device(self.previous)
+
+
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw handle of the device's current stream (without building a ``torch.cuda.Stream``, 3 us)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)

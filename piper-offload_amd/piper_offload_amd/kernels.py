@@ -64,11 +64,12 @@ def _run(name: str, device: torch.device, ws_bytes: int, *args: object) -> None:
     The workspace comes from torch's caching allocator on the same stream, so
     releasing it after the (asynchronous) launch is stream-ordered.
     """
-    handle = L.lib()
-    with torch.cuda.device(device):
+    entry = getattr(L.lib(), name)
+    with L.on_device(device):
         ws = L.workspace(ws_bytes, device)
-        rc = getattr(handle, name)(*args, L.aligned_ptr(ws), ws_bytes, L.stream_ptr(device))
-    L.check(rc)
+        rc = entry(*args, L.aligned_ptr(ws), ws_bytes, L.stream_ptr(device))
+    if rc:
+        L.check(rc)
 
 
 def _factors(b: torch.Tensor, a: torch.Tensor, rows: int, cols: int, label: str) -> tuple[torch.Tensor, torch.Tensor]:
@@ -155,7 +156,7 @@ def merge_int8_lora_into(
             raise ValueError("HIP INT8 merge requires contiguous storage.")
     lora = L.lora_struct(b, a, strength)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, a.shape[0])
+    ws_bytes = L.workspace_size(rows, cols, a.shape[0])
     _run("lm_int8_merge", device, ws_bytes,
          _ptr(qdata), _ptr(scale), _ptr(zero_point), _ptr(out_qdata), _ptr(out_scale), _ptr(out_zero_point),
          rows, cols, group, L.torch_dtype_id(scale.dtype), int(asymmetric), int(reduce_range),
@@ -195,7 +196,7 @@ def requantize_int8(dense: torch.Tensor, block_size: tuple[int, int], *, scale_d
     out_z = torch.empty(qshape, device=device, dtype=torch.int8)
     assert out_s.numel() == nq
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, 0)
+    ws_bytes = L.workspace_size(rows, cols, 0)
     _run("lm_int8_requant", device, ws_bytes, _ptr(dense), L.torch_dtype_id(dense.dtype), _ptr(out_q), _ptr(out_s),
          _ptr(out_z), rows, cols, group, L.torch_dtype_id(scale_dtype), int(asymmetric), int(reduce_range),
          ctypes.byref(rnd))
@@ -215,7 +216,7 @@ def dequantize_int8(qdata: torch.Tensor, scale: torch.Tensor, zero_point: torch.
     if lora is not None:
         b, a = _factors(lora[0], lora[1], rows, cols, "INT8")
         lora_s, rank = L.lora_struct(b, a, lora[2]), a.shape[0]
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, rank)
+    ws_bytes = L.workspace_size(rows, cols, rank)
     _run("lm_int8_dequant", device, ws_bytes, _ptr(qdata), _ptr(scale.contiguous()),
          _ptr(None if zero_point is None else zero_point.contiguous()), rows, cols, group,
          L.torch_dtype_id(scale.dtype), None if lora_s is None else ctypes.byref(lora_s), _ptr(out),
@@ -265,7 +266,7 @@ def merge_float8_lora_into(qdata: torch.Tensor, scale: torch.Tensor, block_size:
     group = _fp8_group((rows, cols), block_size, scale)
     lora = L.lora_struct(b, a, strength)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, a.shape[0])
+    ws_bytes = L.workspace_size(rows, cols, a.shape[0])
     _run("lm_fp8_merge", device, ws_bytes, _ptr(qdata), _ptr(scale), _ptr(out_qdata), _ptr(out_scale), rows, cols,
          group, L.torch_dtype_id(qdata.dtype), ctypes.byref(lora), ctypes.byref(rnd))
 
@@ -301,7 +302,7 @@ def requantize_float8(dense: torch.Tensor, block_size: tuple[int, int], *, fp8_d
     out_s = torch.empty(sshape, device=device, dtype=torch.float32)
     group = _fp8_group((rows, cols), block_size, out_s)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, 0)
+    ws_bytes = L.workspace_size(rows, cols, 0)
     _run("lm_fp8_requant", device, ws_bytes, _ptr(dense), L.torch_dtype_id(dense.dtype), _ptr(out_q), _ptr(out_s),
          rows, cols, group, L.torch_dtype_id(fp8_dtype), ctypes.byref(rnd))
     return out_q, out_s
@@ -319,7 +320,7 @@ def dequantize_float8(qdata: torch.Tensor, scale: torch.Tensor, block_size: tupl
     if lora is not None:
         b, a = _factors(lora[0], lora[1], rows, cols, "scaled-FP8")
         lora_s, rank = L.lora_struct(b, a, lora[2]), a.shape[0]
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, rank)
+    ws_bytes = L.workspace_size(rows, cols, rank)
     _run("lm_fp8_dequant", device, ws_bytes, _ptr(qdata), _ptr(scale.contiguous()), rows, cols, group,
          L.torch_dtype_id(qdata.dtype), None if lora_s is None else ctypes.byref(lora_s), _ptr(out),
          L.torch_dtype_id(dtype))
@@ -361,7 +362,7 @@ def merge_nvfp4_lora_into(qdata: torch.Tensor, scale: torch.Tensor, per_tensor_s
         raise ValueError("HIP NVFP4 merge expects one float32 per-tensor scale.")
     lora = L.lora_struct(b, a, strength)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, a.shape[0])
+    ws_bytes = L.workspace_size(rows, cols, a.shape[0])
     _run("lm_nvfp4_merge", device, ws_bytes, _ptr(qdata), _ptr(scale.view(torch.uint8)), _ptr(per_tensor_scale),
          _ptr(out_qdata), _ptr(out_scale.view(torch.uint8)), _ptr(out_per_tensor_scale), rows, cols,
          int(is_swizzled_scales), ctypes.byref(lora), ctypes.byref(rnd))
@@ -389,7 +390,7 @@ def requantize_nvfp4(dense: torch.Tensor, *, two_level: bool = True, swizzled: b
     out_s = torch.zeros(_nvfp4_scale_shape(rows, cols, swizzled), device=device, dtype=torch.float8_e4m3fn)
     out_pts = torch.empty((), device=device, dtype=torch.float32) if two_level else None
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, 0)
+    ws_bytes = L.workspace_size(rows, cols, 0)
     _run("lm_nvfp4_requant", device, ws_bytes, _ptr(dense), L.torch_dtype_id(dense.dtype), _ptr(out_q),
          _ptr(out_s.view(torch.uint8)), _ptr(out_pts), rows, cols, int(swizzled), ctypes.byref(rnd))
     return out_q, out_s, out_pts
@@ -405,7 +406,7 @@ def dequantize_nvfp4(qdata: torch.Tensor, scale: torch.Tensor, per_tensor_scale:
     if lora is not None:
         b, a = _factors(lora[0], lora[1], rows, cols, "NVFP4")
         lora_s, rank = L.lora_struct(b, a, lora[2]), a.shape[0]
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, rank)
+    ws_bytes = L.workspace_size(rows, cols, rank)
     _run("lm_nvfp4_dequant", device, ws_bytes, _ptr(qdata.contiguous()), _ptr(scale.contiguous().view(torch.uint8)),
          _ptr(per_tensor_scale), rows, cols, int(swizzled), None if lora_s is None else ctypes.byref(lora_s),
          _ptr(out), L.torch_dtype_id(dtype))
@@ -469,7 +470,7 @@ def merge_mx_lora_(qdata: torch.Tensor, scale: torch.Tensor, elem_dtype: torch.d
     b, a = _factors(b, a, rows, cols, "MX")
     lora = L.lora_struct(b, a, strength)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, rank)
+    ws_bytes = L.workspace_size(rows, cols, rank)
     _run("lm_mx_merge", device, ws_bytes, _ptr(qdata), _ptr(scale), rows, cols, fmt, int(scaling_mode),
          int(swizzled), ctypes.byref(lora), ctypes.byref(rnd))
 
@@ -484,7 +485,7 @@ def requantize_mx(dense: torch.Tensor, elem_dtype: torch.dtype, *, scaling_mode:
                         dtype=torch.uint8 if fmt == L.LM_E2M1 else elem_dtype)
     out_s = torch.zeros(_mx_scale_shape(rows, cols, swizzled), device=device, dtype=torch.uint8)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, 0)
+    ws_bytes = L.workspace_size(rows, cols, 0)
     _run("lm_mx_requant", device, ws_bytes, _ptr(dense), L.torch_dtype_id(dense.dtype), _ptr(out_q), _ptr(out_s),
          rows, cols, fmt, int(scaling_mode), int(swizzled), ctypes.byref(rnd))
     return out_q, out_s
@@ -501,7 +502,7 @@ def dequantize_mx(qdata: torch.Tensor, scale: torch.Tensor, elem_dtype: torch.dt
     if lora is not None:
         b, a = _factors(lora[0], lora[1], rows, cols, "MX")
         lora_s, rank = L.lora_struct(b, a, lora[2]), a.shape[0]
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, rank)
+    ws_bytes = L.workspace_size(rows, cols, rank)
     _run("lm_mx_dequant", device, ws_bytes, _ptr(qdata.contiguous()), _ptr(scale.contiguous()), rows, cols, fmt,
          int(swizzled), None if lora_s is None else ctypes.byref(lora_s), _ptr(out), L.torch_dtype_id(dtype))
     return out
@@ -529,7 +530,7 @@ def merge_q8_0_lora(packed: torch.Tensor, b: torch.Tensor, a: torch.Tensor, stre
     out = torch.empty_like(packed) if out is None else out
     lora = L.lora_struct(b, a, strength)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, a.shape[0])
+    ws_bytes = L.workspace_size(rows, cols, a.shape[0])
     _run("lm_q8_0_merge", device, ws_bytes, _ptr(packed), _ptr(out), rows, cols, ctypes.byref(lora),
          ctypes.byref(rnd))
     return out
@@ -543,7 +544,7 @@ def requantize_q8_0(dense: torch.Tensor, *, rounding_seed: int | None = None) ->
         raise ValueError("Q8_0 requires columns divisible by 32.")
     out = torch.empty((rows, cols // _Q8_0_BLOCK * _Q8_0_BYTES), device=device, dtype=torch.uint8)
     rnd = L.rounding_struct(rounding_seed)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, 0)
+    ws_bytes = L.workspace_size(rows, cols, 0)
     _run("lm_q8_0_requant", device, ws_bytes, _ptr(dense), L.torch_dtype_id(dense.dtype), _ptr(out), rows, cols,
          ctypes.byref(rnd))
     return out
@@ -593,7 +594,7 @@ def dequantize_gguf(data: torch.Tensor, quant_type: int, *, dtype: torch.dtype =
             raise ValueError("GGUF dequant with LoRA factors supports Q8_0 only.")
         b, a = _factors(lora[0], lora[1], rows, cols, "GGUF")
         lora_s, rank = L.lora_struct(b, a, lora[2]), a.shape[0]
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, rank) if lora is not None else 0
+    ws_bytes = L.workspace_size(rows, cols, rank) if lora is not None else 0
     _run("lm_gguf_dequant", device, ws_bytes, _ptr(raw), int(quant_type), rows, cols,
          None if lora_s is None else ctypes.byref(lora_s), _ptr(out), L.torch_dtype_id(dtype))
     return out
@@ -612,5 +613,5 @@ def merge_dense_lora_(weight: torch.Tensor, b: torch.Tensor, a: torch.Tensor, st
     rows, cols = weight.shape
     b, a = _factors(b, a, rows, cols, "dense")
     lora = L.lora_struct(b, a, strength)
-    ws_bytes = L.load_library().lm_workspace_size(rows, cols, a.shape[0])
+    ws_bytes = L.workspace_size(rows, cols, a.shape[0])
     _run("lm_dense_merge", device, ws_bytes, _ptr(weight), rows, cols, weight.stride(0), ctypes.byref(lora))

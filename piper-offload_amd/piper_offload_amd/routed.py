@@ -94,7 +94,7 @@ def routed_residual(x: torch.Tensor, factors: Sequence[RoutedFactor], output: to
         return out.view(output.shape)
     handle = L.lib()
     ws_bytes = handle.lm_routed_workspace_size(t, k, arr, len(factors))
-    with torch.cuda.device(device):
+    with L.on_device(device):
         # at most 16 tokens need no workspace (one launch, LDS only)
         ws = L.workspace(ws_bytes, device) if ws_bytes else None
         rc = handle.lm_routed_residual(x2.data_ptr(), y2.data_ptr(), out.data_ptr(), t, k, n, L.torch_dtype_id(dtype),
