@@ -28,6 +28,10 @@
 typedef uint32_t lm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t lm_u32x4 __attribute__((ext_vector_type(4)));
 
+// 16 bytes at any address: one global_load / global_store_dwordx4 (the hardware
+// takes unaligned vector accesses), for rows whose length is no multiple of 16
+typedef uint32_t lm_u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef _Float16 v4f16 __attribute__((ext_vector_type(4)));
 typedef float v4f32 __attribute__((ext_vector_type(4)));
@@ -435,11 +439,33 @@ DEV void sr_bits(uint64_t seed, uint64_t idx0, uint32_t (&h)[SPAN]) {
       for (int j = 0; j < 8; ++j) h[gi * 8 + j] = sr_h_of(c, j);
     }
   } else {
-    for (int j = 0; j < SPAN; ++j) {
-      uint64_t idx = idx0 + j;
+    // the span lies in SPAN / 8 + 1 Philox blocks (rows of odd length): their
+    // halfwords as one stream, two to a word with the earlier one low, shifted
+    // down by the idx0 % 8 that come before the span
+    // (masks rather than selects: selects of array elements went to scratch memory)
+    constexpr int NW = SPAN / 2 + 4;
+    uint32_t w[NW], v[NW - 2], x[NW - 3];
+#pragma unroll
+    for (int gi = 0; gi < SPAN / 8 + 1; ++gi) {
       uint32_t c[4];
-      philox_sr(idx >> 3, seed, c);
-      h[j] = sr_h_of(c, (int)(idx & 7));
+      philox_sr((idx0 >> 3) + gi, seed, c);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t y = (k & 1) ? ~c[k] : c[k];
+        w[4 * gi + k] = __builtin_amdgcn_alignbit(y, y, 16);
+      }
+    }
+    const uint32_t m4 = 0u - (((uint32_t)idx0 >> 2) & 1u), m2 = 0u - (((uint32_t)idx0 >> 1) & 1u);
+#pragma unroll
+    for (int t = 0; t < NW - 2; ++t) v[t] = (m4 & w[t + 2]) | (~m4 & w[t]);
+#pragma unroll
+    for (int t = 0; t < NW - 3; ++t) x[t] = (m2 & v[t + 1]) | (~m2 & v[t]);
+    const uint32_t sh = ((uint32_t)idx0 & 1u) * 16u;
+#pragma unroll
+    for (int t = 0; t < SPAN / 2; ++t) {
+      const uint32_t y = __builtin_amdgcn_alignbit(x[t + 1], x[t], sh);
+      h[2 * t] = y & 0xffffu;
+      h[2 * t + 1] = y >> 16;
     }
   }
 }

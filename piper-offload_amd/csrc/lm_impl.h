@@ -402,11 +402,11 @@ __device__ __forceinline__ void row_merged_tile(const RowArgs& a, int64_t row, b
                                                 int64_t mt_col0, const v4i16 (&bop)[NKC], float s_in, float z_in,
                                                 float (&m)[16]) {
   const int64_t N = a.N;
-  const bool full = rok && (c0 + 16 <= N) && ((N & 15) == 0);
+  const bool full = rok && (c0 + 16 <= N);  // any row length: unaligned 16-byte accesses
   if constexpr (FROM_DENSE) {
     if (full) {
-      const uint4* p = (const uint4*)(a.dense + row * N + c0);
-      uint4 w0 = p[0], w1 = p[1];
+      const LM_GLOBAL lm_u32x4_any* p = (const LM_GLOBAL lm_u32x4_any*)(a.dense + row * N + c0);
+      const lm_u32x4 w0 = p[0], w1 = p[1];
       uint32_t w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
       for (int j = 0; j < 16; ++j) m[j] = val_dt<CD>((j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu));
@@ -418,7 +418,7 @@ __device__ __forceinline__ void row_merged_tile(const RowArgs& a, int64_t row, b
   } else {
     uint32_t w[4];
     if (full) {
-      uint4 v = *(const uint4*)((const uint8_t*)a.q + row * N + c0);
+      const lm_u32x4 v = *(const LM_GLOBAL lm_u32x4_any*)((const uint8_t*)a.q + row * N + c0);
       w[0] = v.x;
       w[1] = v.y;
       w[2] = v.z;
@@ -459,7 +459,7 @@ __device__ __forceinline__ void row_quant_store(const RowArgs& a, int64_t row, b
                                                 const float (&m)[16]) {
   const int64_t N = a.N;
   if (!rok || c0 >= N) return;
-  const bool full = (c0 + 16 <= N) && ((N & 15) == 0);
+  const bool full = c0 + 16 <= N;
   uint32_t h[16];
   if constexpr (SR) sr_bits<16>(a.seed, (uint64_t)(row * N + c0), h);
   uint32_t w[4];
@@ -506,7 +506,9 @@ __device__ __forceinline__ void row_quant_store(const RowArgs& a, int64_t row, b
   }
   uint8_t* dst = (uint8_t*)a.q_out + row * N + c0;
   if (full) {
-    *(uint4*)dst = make_uint4(w[0], w[1], w[2], w[3]);
+    const lm_u32x4 v = {w[0], w[1], w[2], w[3]};
+    *(LM_GLOBAL lm_u32x4_any*)dst = v;
+    asm volatile("s_nop 1" ::"v"(v) : "memory");  // (store_b128_guarded)
   } else {
     for (int j = 0; j < 16 && c0 + j < N; ++j) dst[j] = (uint8_t)(w[j >> 2] >> (8 * (j & 3)));
   }
@@ -1337,8 +1339,8 @@ __device__ __forceinline__ void blk_load_base(const BlkArgs& a, int64_t row, boo
     }
   } else if constexpr (F == B_DENSE) {
     const uint16_t* p = (const uint16_t*)a.q + row * a.ld + c0;
-    if (c0 + 16 <= N && (a.ld & 7) == 0) {
-      uint4 w0 = ((const uint4*)p)[0], w1 = ((const uint4*)p)[1];
+    if (c0 + 16 <= N) {
+      const lm_u32x4 w0 = ((const LM_GLOBAL lm_u32x4_any*)p)[0], w1 = ((const LM_GLOBAL lm_u32x4_any*)p)[1];
       uint32_t w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
       for (int j = 0; j < 16; ++j) base[j] = val_dt<CD>((j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu));
@@ -1352,10 +1354,9 @@ __device__ __forceinline__ void blk_load_base(const BlkArgs& a, int64_t row, boo
     float z = 0.0f;
     if constexpr (F == B_INT8) z = a.aux ? (float)((const int8_t*)a.aux)[qi] : 0.0f;
     const uint8_t* p = (const uint8_t*)a.q + row * N + c0;
-    const bool full = (c0 + 16 <= N) && ((N & 15) == 0);
     uint32_t w[4];
-    if (full) {
-      uint4 v = *(const uint4*)p;
+    if (c0 + 16 <= N) {
+      const lm_u32x4 v = *(const LM_GLOBAL lm_u32x4_any*)p;
       w[0] = v.x;
       w[1] = v.y;
       w[2] = v.z;
@@ -1500,12 +1501,16 @@ __device__ __forceinline__ void blk_store(const BlkArgs& a, int64_t row, int64_t
     }
   } else if constexpr (F == B_DENSE) {
     uint16_t* p = (uint16_t*)a.q_out + row * a.ld + c0;
-    if (c0 + 16 <= N && (a.ld & 7) == 0) {
-      uint32_t w[8];
+    if (c0 + 16 <= N) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) w[k] = (uint32_t)bits_dt<CD>(m[2 * k]) | ((uint32_t)bits_dt<CD>(m[2 * k + 1]) << 16);
-      ((uint4*)p)[0] = make_uint4(w[0], w[1], w[2], w[3]);
-      ((uint4*)p)[1] = make_uint4(w[4], w[5], w[6], w[7]);
+      for (int i = 0; i < 2; ++i) {
+        lm_u32x4 w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          w[k] = (uint32_t)bits_dt<CD>(m[8 * i + 2 * k]) | ((uint32_t)bits_dt<CD>(m[8 * i + 2 * k + 1]) << 16);
+        ((LM_GLOBAL lm_u32x4_any*)p)[i] = w;
+        asm volatile("s_nop 1" ::"v"(w) : "memory");  // (store_b128_guarded)
+      }
     } else {
       for (int j = 0; j < 16 && c0 + j < N; ++j) p[j] = bits_dt<CD>(m[j]);
     }
