@@ -30,8 +30,9 @@
  *    device memory (scratch comes from the caller's `workspace`, sized by
  *    lm_workspace_size()) and none synchronizes: every call is asynchronous
  *    on `stream`.  The *_stack entry points copy their descriptor tables
- *    into the workspace through pinned host staging owned by the library,
- *    so the caller's item array may be reused as soon as the call returns;
+ *    into the workspace as kernel arguments or, when large, through pinned
+ *    host staging owned by the library, so the caller's item array may be
+ *    reused as soon as the call returns;
  *    the workspace must stay allocated until the stream has run the call
  *    (stream-ordered allocators such as torch's satisfy this).
  *  - Return value: LM_OK or an lm_status; lm_last_error() returns a
