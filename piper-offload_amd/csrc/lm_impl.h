@@ -747,9 +747,11 @@ __device__ __forceinline__ void fast_tile_delta(const v4i16 (&aop)[4][NKC], cons
 // bf16-rounded values is bf16r of it)
 // LUT: INT8 only, lut = the lane's row of bf16(RN(q s)) for the 256 code
 // bytes (rows_fast_body), read instead of converting and scaling each code
-template <int KIND, bool AMAX = true, bool LUT = false>
+// ZP: INT8 only, the codes' zero point z is subtracted
+template <int KIND, bool AMAX = true, bool LUT = false, bool ZP = false>
 __device__ __forceinline__ void fast_merge_vals(const RowArgs& a, const uint4& raw, const float (&d)[16], float s_in,
-                                                float (&m)[16], float& amax, const float* lut = nullptr) {
+                                                float (&m)[16], float& amax, const float* lut = nullptr,
+                                                float z = 0.0f) {
   static_assert(!LUT || KIND == K_INT8, "the dequant table is for INT8 codes");
   const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -766,8 +768,14 @@ __device__ __forceinline__ void fast_merge_vals(const RowArgs& a, const uint4& r
     } else if constexpr (KIND == K_INT8) {
       // signed byte -> fp32 is one sign-extending SDWA convert; RN(q * s)
       const int b0 = (2 * k) & 3, b1 = (2 * k + 1) & 3;
-      x0 = (float)(int8_t)(word >> (8 * b0)) * s_in;
-      x1 = (float)(int8_t)(word >> (8 * b1)) * s_in;
+      x0 = (float)(int8_t)(word >> (8 * b0));
+      x1 = (float)(int8_t)(word >> (8 * b1));
+      if constexpr (ZP) {
+        x0 -= z;
+        x1 -= z;
+      }
+      x0 *= s_in;
+      x1 *= s_in;
     } else {
       const v2f32 c = (k & 1) ? fp8_decode_pair<FmtLimit<KIND>::fmt, true>(word)
                               : fp8_decode_pair<FmtLimit<KIND>::fmt, false>(word);

@@ -9,12 +9,13 @@
 // tile's A^T operands and walks TPW tiles; the workgroup's 4 waves take
 // neighbouring tiles):
 //   amax   merge, max |bf16(merged)|, one partial per workgroup in the
-//          workspace; the first workgroup copies the input scale to red[1];
+//          workspace; the first workgroup copies the input scale to red[1]
+//          and the zero point, if there is one, to red[2];
 //   quant  each workgroup reduces the partials (a few KB from L2), merges
 //          again (the same MFMA chains and arithmetic, so the values are
 //          those the amax pass reduced), quantizes and stores; the first
-//          stores the scale.  It reads the input scale from red[1], since
-//          the output may alias it.
+//          stores the scale.  It reads the input scale and zero point from
+//          red[1] and red[2], since the outputs may alias them.
 // The codes are read twice, the second time from the last-level cache where
 // they fit.  What bounds the passes is the latency of their loads and the
 // merge arithmetic.  Atomics do not pay here: the waves of one generation end
@@ -22,7 +23,8 @@
 // [8192, 4096] rank 32: 57.9 us with one conditional atomic per wave, 30.5 with
 // partials).  Per call, against the k_blocks passes that these layouts took
 // before: FP8 [13800, 5120] rank 32 157 -> 62 us, [14336, 4096] rank 16
-// stochastic 141 -> 47, [8192, 8192] rank 64 199 -> 73.
+// stochastic 141 -> 47, [8192, 8192] rank 64 199 -> 73; INT8 [14336, 4096] rank
+// 16 132 -> 42, with a zero point to subtract 135 -> 42.
 #include "lm_tensor.h"
 
 namespace {
@@ -44,10 +46,13 @@ __global__ __launch_bounds__(TT_NW * 64) void k_tensor_pass(RowArgs a, int wg_pe
   const bool first = unit == 0 && threadIdx.x == 0;
   LM_GLOBAL uint32_t* red = (LM_GLOBAL uint32_t*)a.red;
   LM_GLOBAL float* part = (LM_GLOBAL float*)(red + TT_PART);  // one maximum per amax workgroup
-  float s_in;
+  // a symmetric INT8 weight may come with a zero point (usually 0), subtracted here; the merged codes have none
+  constexpr bool ZP = KIND == K_INT8;
+  float s_in, z_in = 0.0f;
   RowQP qp = {0.0f, 0.0f, 0.0f, 0.0f};
   if constexpr (QUANT) {
     s_in = u2f(red[1]);
+    if (ZP && a.zp) z_in = u2f(red[2]);
     float mx = 0.0f;
     for (int i = threadIdx.x; i < npart; i += TT_NW * 64) mx = __builtin_fmaxf(mx, part[i]);
     mx = wave_max(mx);
@@ -66,6 +71,10 @@ __global__ __launch_bounds__(TT_NW * 64) void k_tensor_pass(RowArgs a, int wg_pe
   } else {
     s_in = *(const LM_GLOBAL float*)a.scale;
     if (first) red[1] = f2u(s_in);
+    if (ZP && a.zp) {
+      z_in = (float)*(const LM_GLOBAL int8_t*)a.zp;
+      if (first) red[2] = f2u(z_in);
+    }
   }
   // a wave without tiles has no steps; it takes part in the barriers
   const int left = (ntiles - t0 + TT_NW - 1) / TT_NW, steps = left < TPW ? left : TPW;
@@ -100,7 +109,7 @@ __global__ __launch_bounds__(TT_NW * 64) void k_tensor_pass(RowArgs a, int wg_pe
       if (rb + 1 < RB) fast_tile_delta<NKC>(aop, bop[rb + 1], d[(rb + 1) & 1]);
       else fast_load_aop<NKC>(L[0], next, aop);
       float m[16];
-      fast_merge_vals<KIND, !QUANT>(a, raw[rb], d[rb & 1], s_in, m, amax);
+      fast_merge_vals<KIND, !QUANT, false, ZP>(a, raw[rb], d[rb & 1], s_in, m, amax, nullptr, z_in);
       raw[rb] = fast_load_codes(L[rb], next);
       if constexpr (QUANT) {
         uint32_t old[8];

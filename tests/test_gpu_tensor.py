@@ -59,3 +59,22 @@ def _case(shape: tuple[int, int], fmt: str, sr: bool, rank: int, dtype: torch.dt
         K.merge_float8_lora_into(q, s, shape, b, a, 0.75, rounding_seed=seed, out_qdata=q, out_scale=s)
     assert np.array_equal(u8_np(q), oq.view(np.uint8))
     assert s.item() == os_[0]
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("shape", [(70, 256), (40, 200)])
+def test_symmetric_with_zero_point(shape: tuple[int, int], in_place: bool) -> None:
+    """A zero point that comes with a symmetric request is subtracted, as in the dense merge; the merged codes have none."""
+    rows, cols = shape
+    rank = 8
+    g = torch.Generator().manual_seed(7)
+    q = torch.randint(-100, 100, (rows, cols), generator=g, dtype=torch.int8).cuda()
+    s, z = torch.full((1, 1), 3e-4, device="cuda"), torch.full((1, 1), 5, dtype=torch.int8, device="cuda")
+    b, a = (t.cuda() for t in lora_factors(rows, cols, rank, rank))
+    dense = K.dequantize_int8(q, s, z, (rows, cols), lora=(b, a, 0.75))
+    oq, os_, _ = O.int8_requant(bf16_np(dense), rows * cols)
+    out_q, out_s, out_z = (q, s, z) if in_place else (torch.empty_like(q), torch.empty_like(s), torch.empty_like(z))
+    K.merge_int8_lora_into(q, s, z, (rows, cols), b, a, 0.75, asymmetric=False, reduce_range=False, rounding_seed=None,
+                           out_qdata=out_q, out_scale=out_s, out_zero_point=out_z)
+    assert np.array_equal(u8_np(out_q), oq.view(np.uint8))
+    assert out_s.item() == os_[0] and out_z.item() == 0
