@@ -73,12 +73,15 @@ DEV void q8_load_raw(const Q8Args& a, const uint32_t (&off)[5], int64_t rg, int 
   for (int i = 0; i < 5; ++i) t.c[i] = *(const LM_GLOBAL lm_u32x2*)(p + off[i]);
 }
 template <int NKC>
-DEV void q8_load_ops(const Q8Args& a, const Q8Lane& L, int64_t rg, int mt, Q8Ops<NKC>& t) {
+DEV void q8_load_aop(const Q8Args& a, const Q8Lane& L, int mt, Q8Ops<NKC>& t) {
   constexpr int RPAD = NKC * 16;
   const LM_GLOBAL uint16_t* at = (const LM_GLOBAL uint16_t*)a.at + (uint32_t)(mt * (128 * RPAD)) + L.aoff;
 #pragma unroll
   for (int k = 0; k < 8; ++k) load_kchunks_g<NKC>(at + 4 * k * RPAD, t.aop[k]);
-  load_kchunks_g<NKC>((const LM_GLOBAL uint16_t*)a.bp + rg * (16 * RPAD) + L.boff, t.bop);
+}
+template <int NKC>
+DEV void q8_load_bop(const Q8Args& a, const Q8Lane& L, int64_t rg, Q8Ops<NKC>& t) {
+  load_kchunks_g<NKC>((const LM_GLOBAL uint16_t*)a.bp + rg * (NKC * 256) + L.boff, t.bop);
 }
 
 // roundf(x) (half away from zero) for |x| < 2^23 in two instructions: adding
@@ -189,46 +192,43 @@ DEV void q8_tile(const Q8Args& a, const Q8Raw& raw, const Q8Ops<NKC>& in, uint8_
 
 constexpr int Q8_NW = 4;
 
-// Wave-persistent: the grid holds exactly the workgroups that fit on the GPU
-// at once, and every wave walks the work items item = gwave, gwave + waves,
-// ... where item = row_group * ntiles + tile (one 16-row x 128-column tile).
-// Single tensors are too small to amortise a wave's launch over a few tiles
-// (a [13824, 5120] tensor is 34560 tiles), so waves stay resident and the last
-// round is at most one tile per wave.  Blocks are independent, so no two
-// waves need each other's results.  The item's row group and tile are
-// wave-uniform and advance by the fixed stride without a division; two
-// register sets alternate so that the next item's loads are in flight while
-// the current one is merged (loads complete in order, so the wait for the
-// current item never waits for the next).  A lane's block starts 2 (g & 1)
+// A wave keeps one 128-column tile, with its A^T operands in registers, and
+// walks down every waves_per_tile-th 16-row group of it (the waves of a
+// workgroup have neighbouring tiles of the same rows).  A tile's A^T operands
+// are rank * 256 bytes against 2176 bytes of codes: read again for every row
+// group, as when waves walked the (row group, tile) items in order, they were 2
+// to 8 times the codes' traffic, from L2, ahead of them in the load queue.
+// Single tensors are too small to amortise a wave's launch over a few row
+// groups (a [13824, 5120] tensor is 34560 items), so as many waves as stay
+// resident share them (q8_fast_run); the last round is at most one item per
+// wave.  Blocks are independent, so no two waves need each other's results.
+// Two register sets alternate so that the next item's loads are in flight
+// while the current one is merged (loads complete in order, so the wait for
+// the current item never waits for the next).  A lane's block starts 2 (g & 1)
 // bytes past a dword boundary in every item (rows are 136 k bytes long), so
 // its window shift is fixed.
-// the second bound is waves per SIMD: rank 16 fits 128 VGPRs (4 waves).
-// Five waves (96 VGPRs) spill and run slower.
+// us per call, three input sets in turn, A^T per item -> per wave, round to
+// nearest / stochastic: [13824, 5120] rank 16 52.9 -> 47.0 / 53.9 -> 50, rank 32
+// 60 -> 46.8 / 60.3 -> 50.8, rank 64 94 -> 53.8 / 99 -> 58.5; [4096, 14336] rank 16
+// 45.6 -> 40.2 / 47.0 -> 42.9.  What is left is memory latency (one item in
+// flight per wave) and the requant arithmetic.
+// The second bound is waves per SIMD: rank 16 round to nearest takes 122 VGPRs
+// (4 waves).  Stochastic needs 136: 3 waves without spills, 50 us, beat 4 with
+// (55) and 4 that read A^T per item (53.7).
 template <int NKC, bool SR>
-constexpr int q8_min_waves() { return NKC == 1 ? 4 : 1; }
+constexpr int q8_min_waves() { return NKC == 1 && !SR ? 4 : 1; }
 
 template <int NKC, bool SR>
-__global__ __launch_bounds__(Q8_NW * 64, (q8_min_waves<NKC, SR>())) void k_q8_fast(Q8Args a) {
+__global__ __launch_bounds__(Q8_NW * 64, (q8_min_waves<NKC, SR>())) void k_q8_fast(Q8Args a, int waves_per_tile) {
   const int lane = threadIdx.x & 63, rl = lane & 15, g = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int RPAD = NKC * 16;
   const int ntiles = (int)(a.N >> 7);
   const int64_t nrg = (a.M + 15) / 16;
-  const int64_t stride = (int64_t)gridDim.x * Q8_NW;
-  const int64_t item0 = (int64_t)blockIdx.x * Q8_NW + wv;
-  if (item0 >= nrg * ntiles) return;
-  int64_t rg = item0 / ntiles;
-  int mt = (int)(item0 - rg * ntiles);
-  const int64_t srg = stride / ntiles;
-  const int smt = (int)(stride - srg * ntiles);
-  auto advance = [&](int64_t& r, int& t) {
-    t += smt;
-    r += srg;
-    if (t >= ntiles) {
-      t -= ntiles;
-      ++r;
-    }
-  };
+  const int64_t gw = (int64_t)blockIdx.x * Q8_NW + wv;
+  int64_t rg = gw / ntiles;
+  const int mt = (int)(gw - rg * ntiles);
+  if (rg >= waves_per_tile || rg >= nrg) return;
   const int64_t rowbytes = a.N / 32 * 34;
   const int sh = 2 * (g & 1);
   const int p = lane & 15;
@@ -261,24 +261,22 @@ __global__ __launch_bounds__(Q8_NW * 64, (q8_min_waves<NKC, SR>())) void k_q8_fa
     const int64_t left = a.M - r * 16;
     q8_tile<NKC, SR>(a, w, t, slot, sh, r * 16 + rl, tile, lane, left < 16 ? (int)left : 16, off, out);
   };
-  // the MFMA operands (L2-resident) are requested at the start of their own
-  // item, then the next item's bytes, into alternating registers (loads
-  // complete in order: waiting for the operands never waits for the next item)
+  // the row group's Bp operand (L2-resident) is requested at the start of its
+  // own item, then the next item's bytes, into alternating registers (loads
+  // complete in order: waiting for the operand never waits for the next item)
   Q8Raw w0, w1;
-  int64_t rg1 = rg;
-  int mt1 = mt;
-  advance(rg1, mt1);
+  Q8Ops<NKC> ops;
+  q8_load_aop<NKC>(a, L, mt, ops);
+  int64_t next = rg + waves_per_tile;
   load_raw(rg, mt, w0);
-#define Q8_STEP(WC, WN)                                   \
-  {                                                       \
-    Q8Ops<NKC> ops;                                       \
-    q8_load_ops<NKC>(a, L, rg, mt, ops);                  \
-    if (rg1 < nrg) load_raw(rg1, mt1, WN);                \
-    run(WC, ops, rg, mt);                                 \
-    if (rg1 >= nrg) break;                                \
-    rg = rg1;                                             \
-    mt = mt1;                                             \
-    advance(rg1, mt1);                                    \
+#define Q8_STEP(WC, WN)                             \
+  {                                                 \
+    q8_load_bop<NKC>(a, L, rg, ops);                \
+    if (next < nrg) load_raw(next, mt, WN);         \
+    run(WC, ops, rg, mt);                           \
+    if (next >= nrg) break;                         \
+    rg = next;                                      \
+    next += waves_per_tile;                         \
   }
   for (;;) {
     Q8_STEP(w0, w1)
@@ -313,15 +311,20 @@ static inline bool q8_fast_ok(int cd, int nkc, int64_t M, int64_t N) {
   return cd == LM_BF16 && nkc > 0 && (N % 128) == 0 && M * N <= (int64_t(1) << 35);
 }
 
+// waves per tile: as many as are resident at once, shared among the tiles; at
+// least 8 (rows of 65536 columns and more), since rounding fewer down would
+// leave up to half of the resident slots empty
 static int q8_fast_run(const Q8Args& a, int nkc, bool sr, hipStream_t st) {
-  const int64_t nitems = ((a.M + 15) / 16) * (a.N >> 7);
+  const int64_t nrg = (a.M + 15) / 16, ntiles = a.N >> 7;
   const dim3 block(Q8_NW * 64);
   TimedLaunch timed("q8", st);
 #define Q8L(SR_)                                                                                           \
   NKC_SWITCH(nkc_bucket(nkc), {                                                                            \
-    const int64_t need = (nitems + Q8_NW - 1) / Q8_NW;                                                     \
-    const unsigned res = q8_resident_grid<NKC_, SR_>();                                                    \
-    hipLaunchKernelGGL((k_q8_fast<NKC_, SR_>), dim3((unsigned)(need < res ? need : res)), block, 0, st, a); \
+    int64_t wpt = (int64_t)q8_resident_grid<NKC_, SR_>() * Q8_NW / ntiles;                                 \
+    if (wpt < 8) wpt = 8;                                                                                  \
+    if (wpt > nrg) wpt = nrg;                                                                              \
+    const int64_t nb = (wpt * ntiles + Q8_NW - 1) / Q8_NW;                                                 \
+    hipLaunchKernelGGL((k_q8_fast<NKC_, SR_>), dim3((unsigned)nb), block, 0, st, a, (int)wpt);              \
   })
   if (sr) { Q8L(true); } else { Q8L(false); }
 #undef Q8L
