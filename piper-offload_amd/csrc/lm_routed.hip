@@ -13,10 +13,12 @@
 //   out    = dt(y + total)
 //
 // At most 16 tokens (decode): one kernel, k_routed_small, and no workspace.
-// Otherwise two:
-// * k_routed_down: MFMA x A^T, one 16-wave workgroup per 16 tokens whose waves
-//   split K and meet in LDS; writes ps = dt(dt(p) s) in the dtype, [T][C * 16]
-//   (C = sum of ceil(r_i / 16) rank chunks);
+// Otherwise two or three:
+// * k_routed_down: MFMA x A^T by 16-wave workgroups whose waves split K and meet
+//   in LDS; writes ps = dt(dt(p) s) in the dtype, [T][C * 16] (C = sum of
+//   ceil(r_i / 16) rank chunks), or, where few tokens leave the GPU idle, the
+//   sums of one of S spans of K (down_plan);
+// * k_routed_finalize (S > 1): adds the spans and writes ps;
 // * k_routed_up: a wave keeps the B operands of one 64-column tile in
 //   registers and walks 16-token tiles: one MFMA chain per factor, the rest
 //   of the rounding chain and one read and one write of y / out: the only
@@ -36,7 +38,9 @@ struct RoutedArgs {
   const uint16_t* y;    // [T, N] (the Linear output)
   uint16_t* out;        // [T, N] (may alias y)
   uint16_t* ps;         // [T][C * 16]: dt(dt(p) s) of each factor's ranks (zero past the rank)
+  float* part;          // S > 1: [S][T][C * 16], the spans' sums
   int64_t T, K, N;
+  int64_t kspan;        // K columns per span of the down projection
   int nf, nchunks;
   int tiles_per_wg;     // token tiles per up workgroup
   const uint16_t* a[RT_MAX_FACTORS];
@@ -103,26 +107,27 @@ __device__ __forceinline__ v4f32 mfma1(const v4i16& a, const v4i16& b, const v4f
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
 }
 
-// grid (token tiles).  The workgroup's 16 waves split K: a round is RT_DU steps
-// of 32 columns per wave, in pairs of 64 neighbouring columns whose rows load as
-// whole cache lines (trade_rows8); all of a round's loads are issued before the
-// MFMAs (K = 4096 is one round).  For rank chunk c the MFMA computes
-// D[r][t] = sum_k A_i[r][k] x[t][k]: lane l holds ranks 16 c' + 4 (l >> 4) + 0..3
-// of token l & 15.  CB chunks share each round's x values; the waves' sums meet
-// in LDS and one thread per (chunk, rank, token) adds them in wave order and
-// rounds.  What bounds it is one trip to memory: with the K range split over
-// 2048 four-wave workgroups, fp32 partials and a kernel that summed them, 4096
-// tokens of K = 4096 took 11.3 + 4.8 us, and this takes 11.
+// grid (token tiles x chunk blocks, S).  A workgroup takes CB rank chunks of 16
+// tokens over one of S spans of K; its 16 waves split the span.  A round is
+// RT_DU steps of 32 columns per wave, in pairs of 64 neighbouring columns whose
+// rows load as whole cache lines (trade_rows8); all of a round's loads are
+// issued before the MFMAs (4096 columns are one round).  For rank chunk c the
+// MFMA computes D[r][t] = sum_k A_i[r][k] x[t][k]: lane l holds ranks 16 c' + 4
+// (l >> 4) + 0..3 of token l & 15.  The CB chunks share each round's x values;
+// the waves' sums meet in LDS and one thread per (chunk, rank, token) adds them
+// in wave order.  With S = 1 it rounds and writes ps; otherwise it writes the
+// span's partial and k_routed_finalize adds the spans.
 constexpr int RT_DNW = 16;
 constexpr int RT_DU = 8;
-// columns k .. k + 63 of rows row0 .. row0 + 15 as two accesses of whole lines;
+constexpr int RT_DSTEP = 64 * RT_DNW;  // columns of one pair per wave: spans are multiples of it
+// columns k .. k + 63 (below ke) of rows row0 .. row0 + 15 as two accesses of whole lines;
 // trade_pair then gives lane (rl, g) columns k + 8 g .. and k + 32 + 8 g .. of row rl
-__device__ __forceinline__ void load_pair(const uint16_t* p, int64_t rows, int64_t cols, int64_t row0, int64_t k, int rl,
-                                          int g, rt_v8i16& v0, rt_v8i16& v1) {
+__device__ __forceinline__ void load_pair(const uint16_t* p, int64_t rows, int64_t cols, int64_t row0, int64_t k,
+                                          int64_t ke, int rl, int g, rt_v8i16& v0, rt_v8i16& v1) {
   const int64_t c = k + 32 * (rl >> 3) + 8 * g;
   const rt_v8i16 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  v0 = c < cols ? load8(p, rows, cols, row0 + (rl & 7), c) : zero;
-  v1 = c < cols ? load8(p, rows, cols, row0 + (rl & 7) + 8, c) : zero;
+  v0 = c < ke ? load8(p, rows, cols, row0 + (rl & 7), c) : zero;
+  v1 = c < ke ? load8(p, rows, cols, row0 + (rl & 7) + 8, c) : zero;
 }
 __device__ __forceinline__ void trade_pair(rt_v8i16& v0, rt_v8i16& v1) {
   lm_u32x4 x = __builtin_bit_cast(lm_u32x4, v0), y = __builtin_bit_cast(lm_u32x4, v1);
@@ -131,52 +136,78 @@ __device__ __forceinline__ void trade_pair(rt_v8i16& v0, rt_v8i16& v1) {
   v1 = __builtin_bit_cast(rt_v8i16, y);
 }
 template <bool HALF, int CB>
-__global__ __launch_bounds__(RT_DNW * 64) void k_routed_down(RoutedArgs a) {
+__global__ __launch_bounds__(RT_DNW * 64) void k_routed_down(RoutedArgs a, FastDiv blocks) {
   constexpr int DT = HALF ? F16 : BF16;
   __shared__ float sh[CB][RT_DNW][256];
   const int lane = threadIdx.x & 63, wave = wave_index(), rl = lane & 15, g = lane >> 4;
-  const int64_t t0 = (int64_t)blockIdx.x * 16;
-  for (int c0 = 0; c0 < a.nchunks; c0 += CB) {
-    v4f32 acc[CB];
+  const uint32_t tile = div_by(blocks, blockIdx.x);
+  const int c0 = (int)(blockIdx.x - tile * blocks.d) * CB;
+  const int64_t t0 = (int64_t)tile * 16;
+  const int64_t kb = (int64_t)blockIdx.y * a.kspan, ke = kb + a.kspan < a.K ? kb + a.kspan : a.K;
+  v4f32 acc[CB];
 #pragma unroll
-    for (int c = 0; c < CB; ++c) acc[c] = (v4f32){0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t k0 = 64 * wave; k0 < a.K; k0 += 32 * RT_DNW * RT_DU) {
-      // loads past K or the rows read zeros
-      rt_v8i16 av[RT_DU], xv[RT_DU];
+  for (int c = 0; c < CB; ++c) acc[c] = (v4f32){0.0f, 0.0f, 0.0f, 0.0f};
+  for (int64_t k0 = kb + 64 * wave; k0 < ke; k0 += 32 * RT_DNW * RT_DU) {
+    // loads past the span or the rows read zeros
+    rt_v8i16 av[RT_DU], xv[RT_DU];
 #pragma unroll
-      for (int u = 0; u < RT_DU; u += 2) load_pair(a.x, a.T, a.K, t0, k0 + (int64_t)u * 32 * RT_DNW, rl, g, xv[u], xv[u + 1]);
+    for (int u = 0; u < RT_DU; u += 2)
+      load_pair(a.x, a.T, a.K, t0, k0 + (int64_t)u * 32 * RT_DNW, ke, rl, g, xv[u], xv[u + 1]);
 #pragma unroll
-      for (int c = 0; c < CB; ++c) {
-        if (c0 + c >= a.nchunks) break;
-        const int i = a.cfac[c0 + c], cc = c0 + c - a.chunk0[i];
+    for (int c = 0; c < CB; ++c) {
+      if (c0 + c >= a.nchunks) break;
+      const int i = a.cfac[c0 + c], cc = c0 + c - a.chunk0[i];
 #pragma unroll
-        for (int u = 0; u < RT_DU; u += 2)
-          load_pair(a.a[i], a.rank[i], a.K, 16 * cc, k0 + (int64_t)u * 32 * RT_DNW, rl, g, av[u], av[u + 1]);
+      for (int u = 0; u < RT_DU; u += 2)
+        load_pair(a.a[i], a.rank[i], a.K, 16 * cc, k0 + (int64_t)u * 32 * RT_DNW, ke, rl, g, av[u], av[u + 1]);
 #pragma unroll
-        for (int u = 0; u < RT_DU; u += 2) {
-          trade_pair(av[u], av[u + 1]);
-          if (c == 0) trade_pair(xv[u], xv[u + 1]);
-          acc[c] = mfma32<HALF>(av[u], xv[u], acc[c]);
-          acc[c] = mfma32<HALF>(av[u + 1], xv[u + 1], acc[c]);
-        }
+      for (int u = 0; u < RT_DU; u += 2) {
+        trade_pair(av[u], av[u + 1]);
+        if (c == 0) trade_pair(xv[u], xv[u + 1]);
+        acc[c] = mfma32<HALF>(av[u], xv[u], acc[c]);
+        acc[c] = mfma32<HALF>(av[u + 1], xv[u + 1], acc[c]);
       }
     }
-#pragma unroll
-    for (int c = 0; c < CB; ++c) *(v4f32*)&sh[c][wave][4 * lane] = acc[c];
-    __syncthreads();
-    for (int o = threadIdx.x; o < CB * 256; o += RT_DNW * 64) {
-      const int c = o >> 8, e = o & 255;  // entry e: token (e >> 2) & 15, rank 4 (e >> 6) + (e & 3)
-      const int64_t t = t0 + ((e >> 2) & 15);
-      if (c0 + c < a.nchunks && t < a.T) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int w = 0; w < RT_DNW; ++w) sum += sh[c][w][e];
-        a.ps[t * (a.nchunks * 16) + (c0 + c) * 16 + 4 * (e >> 6) + (e & 3)] =
-            bits_dt<DT>(round_dt<DT>(round_dt<DT>(sum) * a.s[a.cfac[c0 + c]]));
-      }
-    }
-    if (c0 + CB < a.nchunks) __syncthreads();  // the sums are read before the next chunks' overwrite them
   }
+#pragma unroll
+  for (int c = 0; c < CB; ++c) *(v4f32*)&sh[c][wave][4 * lane] = acc[c];
+  __syncthreads();
+  for (int o = threadIdx.x; o < CB * 256; o += RT_DNW * 64) {
+    const int c = o >> 8, e = o & 255;  // entry e: token (e >> 2) & 15, rank 4 (e >> 6) + (e & 3)
+    const int64_t t = t0 + ((e >> 2) & 15);
+    if (c0 + c < a.nchunks && t < a.T) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int w = 0; w < RT_DNW; ++w) sum += sh[c][w][e];
+      const int64_t at = t * (a.nchunks * 16) + (c0 + c) * 16 + 4 * (e >> 6) + (e & 3);
+      if (gridDim.y > 1) a.part[(int64_t)blockIdx.y * a.T * (a.nchunks * 16) + at] = sum;
+      else a.ps[at] = bits_dt<DT>(round_dt<DT>(round_dt<DT>(sum) * a.s[a.cfac[c0 + c]]));
+    }
+  }
+}
+
+// S > 1: one thread per (token, chunk, 4 ranks) adds the S partials in span
+// order and applies p_i = dt(p), ps_i = dt(p_i s_i)
+template <bool HALF>
+__global__ __launch_bounds__(256) void k_routed_finalize(RoutedArgs a, int S) {
+  constexpr int DT = HALF ? F16 : BF16;
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x, n = a.T * a.nchunks * 4;
+  if (q >= n) return;
+  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int sp = 0; sp < S; ++sp) {
+    const float4 w = ((const float4*)a.part)[sp * n + q];
+    v[0] += w.x;
+    v[1] += w.y;
+    v[2] += w.z;
+    v[3] += w.w;
+  }
+  const float s = a.s[a.cfac[(int)(q % (a.nchunks * 4)) >> 2]];
+  uint32_t w[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    w[h] = (uint32_t)bits_dt<DT>(round_dt<DT>(round_dt<DT>(v[2 * h]) * s)) |
+           ((uint32_t)bits_dt<DT>(round_dt<DT>(round_dt<DT>(v[2 * h + 1]) * s)) << 16);
+  ((uint2*)a.ps)[q] = make_uint2(w[0], w[1]);
 }
 
 // Columns of the up kernels: in a 64-column tile lane group g = lane >> 4 holds
@@ -225,7 +256,7 @@ __device__ __forceinline__ void up_store(const RoutedArgs& a, int64_t t, int64_t
 // grid (column-tile groups, token groups).  Every wave owns one 64-column
 // tile: its B operands (all rank chunks, CMAX at most) stay in registers
 // while it walks the token tiles of its token group.  Per token tile it needs
-// the partial sums of p (L2) and the Linear output y (HBM); both are
+// its rows of ps (L2) and the Linear output y (HBM); both are
 // requested one token tile ahead, after the current tile's own loads, so that
 // waiting for the current tile never waits for the prefetch (loads complete
 // in order).
@@ -378,7 +409,7 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up1(RoutedArgs a) {
 }
 
 // ---- one launch for at most 16 tokens (decode) ---------------------------------
-// Three launches cost more than their work when T is small.  Here every
+// Several launches cost more than their work when T is small.  Here every
 // workgroup computes the whole down projection of the one token tile (its
 // RT_SNW waves split K, one round of RT_DU loads each at K = 4096; the sums
 // meet in LDS), applies the first two roundings into LDS, then each wave
@@ -491,17 +522,51 @@ __global__ __launch_bounds__(RT_SNW * 64) void k_routed_small(RoutedArgs a) {
   if (tok) up_store<DT>(a, t, mt, g, vec, y0, y1, total);
 }
 
+// How the down projection is shared out: CB rank chunks per workgroup, S spans
+// of K.  A workgroup is bound by the latency of its rounds (about 4 us for 4096
+// columns of one chunk), so up to one per CU each more takes work off the
+// others: chunk blocks (a larger block shares its x) and spans (which cost a
+// launch and S partials of p).  Long spans take the largest block that reaches
+// RT_DWG workgroups with them; where that would take spans of less than 3 steps
+// (3072 columns), smaller blocks come first (1024 tokens, rank 64: K 14336 CB 4
+// and S 4 41.6 us, CB 1 and S 1 45.8; K 4096 27.5 and 27.0).  Per call, K -> 4096,
+// one workgroup per 16 tokens -> this: 17 tokens, rank 16, K 4096 12.5 -> 9.4 us;
+// four rank-64 factors, K 4096 94 -> 26, K 14336 277 -> 30; 256 tokens, rank 64,
+// K 14336 71 -> 20; 1024 tokens, rank 64, K 4096 37.1 -> 26.8.  More than RT_DWG
+// workgroups do not pay (2048 tokens, K 4096: rank 16 20.0 us with 128 or 256,
+// 21.7 with 512; rank 64 43.6 with 256, 48.4 with 512).
+constexpr int64_t RT_DWG = 256;
+constexpr int64_t RT_MAX_S = 16;
+struct DownPlan {
+  int cb, blocks;
+  int64_t S, kspan;
+};
+DownPlan down_plan(int64_t T, int64_t K, int chunks) {
+  const int64_t tiles = (T + 15) / 16, steps = (K + RT_DSTEP - 1) / RT_DSTEP;
+  DownPlan d;
+  d.cb = chunks > 2 ? 4 : chunks;
+  for (;; d.cb /= 2) {
+    d.blocks = (chunks + d.cb - 1) / d.cb;
+    d.S = RT_DWG / (tiles * d.blocks);
+    if (d.S <= (steps < 6 ? 1 : steps / 3) || d.cb == 1) break;
+  }
+  if (d.S > RT_MAX_S) d.S = RT_MAX_S;
+  if (d.S < 1) d.S = 1;
+  d.kspan = (steps + d.S - 1) / d.S * RT_DSTEP;
+  d.S = (K + d.kspan - 1) / d.kspan;
+  return d;
+}
+
 }  // namespace
 
 extern "C" size_t lm_routed_workspace_size(int64_t T, int64_t K, const lm_routed_factor* factors, int32_t count) {
   if (T <= 16) return 0;  // the single-launch path keeps everything in LDS
-  (void)K;
   int chunks = 0;
   for (int i = 0; i < count && factors; ++i) chunks += (factors[i].rank + 15) / 16;
-  // ps in the dtype, and room for p in fp32: the size that this entry point has
-  // promised callers since p was summed over launches
+  if (chunks < 1 || K < 1) return 256;  // (lm_routed_residual refuses these)
+  const DownPlan d = down_plan(T, K, chunks);
   const size_t tt = (size_t)T * (size_t)chunks * 16;
-  return align256(tt * sizeof(float)) + align256(tt * sizeof(uint16_t));
+  return align256(tt * sizeof(uint16_t)) + (d.S > 1 ? align256((size_t)d.S * tt * sizeof(float)) : 0);
 }
 
 extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64_t T, int64_t K, int64_t N,
@@ -545,7 +610,10 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
   a.x = (const uint16_t*)x;
   a.y = (const uint16_t*)y;
   a.out = (uint16_t*)out;
+  const DownPlan d = down_plan(T, K, chunks);
   a.ps = (uint16_t*)workspace;
+  a.part = (float*)((uint8_t*)workspace + align256((size_t)T * (size_t)chunks * 16 * sizeof(uint16_t)));
+  a.kspan = d.kspan;
   a.T = T;
   a.K = K;
   a.N = N;
@@ -561,7 +629,7 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
   if (tgroups < 1) tgroups = 1;
   a.tiles_per_wg = (int)((tiles + tgroups - 1) / tgroups);
   tgroups = (tiles + a.tiles_per_wg - 1) / a.tiles_per_wg;
-  if (tiles > 0x7fffffff || tgroups > 65535 || colgroups > 0x7fffffff)
+  if (tiles * d.blocks > 0x7fffffff || tgroups > 65535 || colgroups > 0x7fffffff)
     return fail(LM_EUNSUPPORTED, "routed residual grid too large");
   hipStream_t st = (hipStream_t)stream;
   TimedLaunch timed("routed", st);
@@ -590,11 +658,14 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
   else if (chunks <= 2) hipLaunchKernelGGL((k_routed_up<H_, 2>), ugrid, block, 0, st, a);           \
   else if (chunks <= 4) hipLaunchKernelGGL((k_routed_up<H_, 4>), ugrid, block, 0, st, a);           \
   else hipLaunchKernelGGL((k_routed_up<H_, RT_MAX_CHUNKS>), ugrid, block, 0, st, a);
-#define RT_DOWN(H_)                                                                            \
-  if (chunks <= 1) hipLaunchKernelGGL((k_routed_down<H_, 1>), dgrid, dblock, 0, st, a);        \
-  else if (chunks <= 2) hipLaunchKernelGGL((k_routed_down<H_, 2>), dgrid, dblock, 0, st, a);   \
-  else hipLaunchKernelGGL((k_routed_down<H_, 4>), dgrid, dblock, 0, st, a);
-  const dim3 dgrid((unsigned)tiles), dblock(RT_DNW * 64);
+  const FastDiv by_blocks = fast_div((uint32_t)d.blocks);
+  const dim3 dgrid((unsigned)(tiles * d.blocks), (unsigned)d.S), dblock(RT_DNW * 64);
+  const dim3 fgrid((unsigned)((T * chunks * 4 + 255) / 256));
+#define RT_DOWN(H_)                                                                                  \
+  if (d.cb == 1) hipLaunchKernelGGL((k_routed_down<H_, 1>), dgrid, dblock, 0, st, a, by_blocks);        \
+  else if (d.cb == 2) hipLaunchKernelGGL((k_routed_down<H_, 2>), dgrid, dblock, 0, st, a, by_blocks);   \
+  else hipLaunchKernelGGL((k_routed_down<H_, 4>), dgrid, dblock, 0, st, a, by_blocks);                  \
+  if (d.S > 1) hipLaunchKernelGGL(k_routed_finalize<H_>, fgrid, dim3(256), 0, st, a, (int)d.S);
   if (dtype == LM_F16) {
     RT_DOWN(true)
     RT_UP(true)

@@ -19,6 +19,7 @@ from torch import nn
 
 import oracle as O
 from helpers import bf16_np
+from piper_offload_amd import _lib as L
 from piper_offload_amd import install_routed_residual_hook, routed_residual
 from piper_offload_amd.routed import RoutedFactor
 
@@ -99,3 +100,18 @@ def test_hook_removal_is_idempotent_and_restores_the_module():
     assert not lin._forward_hooks and not lin._forward_pre_hooks
     x = torch.randn(2, 4)
     assert torch.equal(lin(x), x @ lin.weight.T)
+
+
+@pytest.mark.parametrize("tokens,k,ranks,spans", [(17, 14336, [64] * 4, 7), (64, 14336, [16], 8), (256, 14336, [64], 4),
+                                                  (17, 4096, [16], 4), (17, 1024, [16], 1), (4096, 14336, [64], 1)])
+def test_few_tokens_share_the_down_projection(tokens, k, ranks, spans):
+    """Few token tiles cannot fill the GPU with one workgroup each: workgroups share K, and the workspace holds their fp32
+    partial sums of p beside p s in the dtype.  Nothing else is asked for."""
+    h = L.load_library()
+    fs = (L.RoutedFactor * len(ranks))()
+    for f, r in zip(fs, ranks):
+        f.rank = r
+    p = tokens * sum((r + 15) // 16 for r in ranks) * 16
+    need = h.lm_routed_workspace_size(tokens, k, fs, len(ranks))
+    assert need <= 2 * p + (16 * 4 * p if spans > 1 else 0) + 512
+    assert need >= 2 * p + (spans * 4 * p if spans > 1 else 0)

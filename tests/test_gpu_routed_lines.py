@@ -4,12 +4,14 @@ round, every chunk count.  Same oracle and bounds as test_gpu_routed.py; the out
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
+import oracle as O
 import test_gpu_routed
 from piper_offload_amd.routed import RoutedFactor, routed_residual
-from test_gpu_routed import _case, _check
+from test_gpu_routed import DT, _bits, _case, _check
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +31,41 @@ def test_lean_up_matches_oracle(T: int, K: int, N: int, rank: int, dtype: torch.
     with torch.no_grad():
         got = routed_residual(x.cuda(), dfs, y.cuda())
     _check(got, x, y, fs, dtype)
+
+
+def _integer_case(T: int, K: int, N: int, ranks: list[int], bias: bool, dtype: torch.dtype, seed: int):
+    """Inputs whose fp32 sums are exact in every order: x, A and b are small integers, so p = x A^T is an integer and p s a
+    multiple of 1/4, both far below 2^16 (|p| < 6 sigma = 6 sqrt(4 K / 3)), and a sum of 64 products p s b spans under 24
+    bits.  Only the roundings to the dtype are left, and those have one order: results equal the oracle bit for bit."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randint(-2, 3, (T, K), generator=g).to(dtype)
+    y = (torch.randn(T, N, generator=g) * 64).to(dtype)
+    fs = [RoutedFactor(torch.randint(-1, 2, (r, K), generator=g).to(dtype),
+                       torch.randint(-2, 3, (N, r), generator=g).to(dtype), [1.0, 0.5, -1.25][i % 3],
+                       torch.randn(N, generator=g).to(dtype) if bias else None) for i, r in enumerate(ranks)]
+    return x, y, fs
+
+
+def _oracle(x, y, fs, dtype) -> torch.Tensor:
+    ref = O.routed_residual(_bits(x), _bits(y), [(_bits(f.a), _bits(f.b), None if f.bias is None else _bits(f.bias),
+                                                  f.strength) for f in fs], dt=DT[dtype])
+    return torch.from_numpy(ref.view(np.int16)).view(dtype)
+
+
+def _cuda(fs):
+    return [RoutedFactor(f.a.cuda(), f.b.cuda(), f.strength, None if f.bias is None else f.bias.cuda()) for f in fs]
+
+
+# The down projection's shares (down_plan): K spans that end inside a step, chunk blocks of 1, 2 and 4 with a last one of
+# fewer chunks, one span and many, more tiles than workgroups wanted.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,K,N,ranks,bias", [(17, 14336, 72, [64, 64, 64, 64], False), (33, 4100, 200, [16], False),
+                                              (130, 3080, 64, [8, 40, 64], True), (300, 9000, 136, [16], False),
+                                              (1030, 2056, 72, [64], False), (1024, 7000, 64, [64], False),
+                                              (1100, 6200, 40, [48, 16, 5], True), (2050, 1024, 64, [16, 16], False),
+                                              (4100, 256, 64, [64], False), (17, 1024, 64, [1], False)])
+def test_down_projection_shares(T: int, K: int, N: int, ranks: list[int], bias: bool, dtype: torch.dtype) -> None:
+    x, y, fs = _integer_case(T, K, N, ranks, bias, dtype, T + K)
+    with torch.no_grad():
+        got = routed_residual(x.cuda(), _cuda(fs), y.cuda())
+    assert torch.equal(got.cpu(), _oracle(x, y, fs, dtype))
