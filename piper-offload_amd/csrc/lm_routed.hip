@@ -621,10 +621,15 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
   a.nchunks = chunks;
   // up kernel: one 64-column tile per wave, token tiles split into groups so
   // that there are about 8192 waves in all (4096 and 16384: 57.5 and 57.7
-  // against 56.3 us for 4096 tokens, 4096 -> 14336, rank 16)
+  // against 56.3 us for 4096 tokens, 4096 -> 14336, rank 16), or 4096 from rank
+  // 64 on, where a wave's B operands (2 KB a chunk) are more than a token tile
+  // of y and out (4 KB): 1024 tokens, 4096 -> 14336, four rank-64 factors 149
+  // against 175 us, 2048 tokens 248 and 259, 2048 tokens, 4096 -> 4096 134 and
+  // 180; rank 48 in three factors 4096 tokens 108 against 92
   const int64_t ntiles = (N + 63) / 64;
   const int64_t colgroups = (ntiles + RT_NW - 1) / RT_NW;
-  int64_t tgroups = (8192 + ntiles - 1) / ntiles;
+  const int64_t waves = chunks < 4 ? 8192 : 4096;
+  int64_t tgroups = (waves + ntiles - 1) / ntiles;
   if (tgroups > tiles) tgroups = tiles;
   if (tgroups < 1) tgroups = 1;
   a.tiles_per_wg = (int)((tiles + tgroups - 1) / tgroups);

@@ -10,6 +10,7 @@ import torch
 
 import oracle as O
 import test_gpu_routed
+from piper_offload_amd import _lib as L
 from piper_offload_amd.routed import RoutedFactor, routed_residual
 from test_gpu_routed import DT, _bits, _case, _check
 
@@ -69,3 +70,37 @@ def test_down_projection_shares(T: int, K: int, N: int, ranks: list[int], bias: 
     with torch.no_grad():
         got = routed_residual(x.cuda(), _cuda(fs), y.cuda())
     assert torch.equal(got.cpu(), _oracle(x, y, fs, dtype))
+
+
+def _through_c_entry(x, fs, y, out) -> None:
+    """lm_routed_residual on GPU tensors, with an output of the caller's (routed_residual allocates its own)."""
+    arr = (L.RoutedFactor * len(fs))()
+    for i, f in enumerate(fs):
+        arr[i].a, arr[i].b, arr[i].bias = f.a.data_ptr(), f.b.data_ptr(), None if f.bias is None else f.bias.data_ptr()
+        arr[i].strength, arr[i].rank = f.strength, f.a.shape[0]
+    (t, k), n, h = x.shape, y.shape[1], L.lib()
+    nbytes = h.lm_routed_workspace_size(t, k, arr, len(fs))
+    ws = L.workspace(nbytes, x.device)
+    L.check(h.lm_routed_residual(x.data_ptr(), y.data_ptr(), out.data_ptr(), t, k, n, L.torch_dtype_id(x.dtype), arr,
+                                 len(fs), L.aligned_ptr(ws), nbytes, L.stream_ptr(x.device)))
+    torch.cuda.synchronize()
+
+
+# Up kernels that walk several token tiles per wave, the last one ragged, and single launches, into another tensor and in
+# place: the output may alias y.  [1033, 14336]: 2 tiles per wave (one factor, and two with a bias), 4 at rank 64 and 80;
+# N % 8 != 0 takes the element-wise stores.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,K,N,ranks,bias", [(1033, 72, 14336, [16], False), (1033, 72, 14336, [8, 24], True),
+                                              (1033, 72, 14336, [64], False), (1033, 72, 14336, [64, 16], False),
+                                              (2100, 40, 8196, [16], False), (47, 96, 200, [48], False),
+                                              (9, 96, 136, [16], False), (16, 96, 100, [16, 24], True)])
+def test_several_token_tiles_and_aliased_output(T: int, K: int, N: int, ranks: list[int], bias: bool,
+                                                dtype: torch.dtype) -> None:
+    x, y, fs = _integer_case(T, K, N, ranks, bias, dtype, T + N)
+    ref, dx, dy, dfs = _oracle(x, y, fs, dtype), x.cuda(), y.cuda(), _cuda(fs)
+    out = torch.empty_like(dy)
+    _through_c_entry(dx, dfs, dy, out)
+    assert torch.equal(out.cpu(), ref)
+    assert torch.equal(dy.cpu(), y)
+    _through_c_entry(dx, dfs, dy, dy)
+    assert torch.equal(dy.cpu(), ref)
