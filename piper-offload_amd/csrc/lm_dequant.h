@@ -131,9 +131,10 @@ DEV void dq_one(const DqArgs& a, int64_t e) {
   else ((uint16_t*)a.out)[e] = (uint16_t)dq_f16_bits(v);
 }
 
-// M N < 2^32 (32-bit chunk and element indices), 8-byte aligned codes (4 for
-// fp4) and 16-byte aligned output (one load and one store per chunk), qparam
-// groups of at least 8 elements (a chunk meets at most two)
+// M N < 2^32 and at most 2^32 swizzled scales (32-bit chunk, element and scale
+// indices), 8-byte aligned codes (4 for fp4) and 16-byte aligned output (one
+// load and one store per chunk), qparam groups of at least 8 elements (a chunk
+// meets at most two)
 template <int F, int DT>
 __global__ __launch_bounds__(DQ_THREADS) void k_dequant(DqArgs a) {
   constexpr int CD = dq_cd<DT>();
@@ -219,8 +220,10 @@ static int launch_dequant(DqArgs a, hipStream_t st) {
   const int64_t n = a.M * a.N;
   const uintptr_t qmask = DqTraits<F>::FP4 ? 3 : 7;
   TimedLaunch timed("todense", st);
-  if (n < (INT64_C(1) << 32) - 8 && ((uintptr_t)a.q & qmask) == 0 && ((uintptr_t)a.out & 15) == 0 &&
-      (DqTraits<F>::BLOCK || a.group >= 8)) {
+  // the swizzled layout pads rows to 128: a few very long rows have far more scale bytes than n / BS
+  const int64_t scales = a.swizzled ? (a.M + 127) / 128 * ((a.N / DqTraits<F>::BS + 3) / 4) * 512 : 0;
+  if (n < (INT64_C(1) << 32) - 8 && scales <= (INT64_C(1) << 32) && ((uintptr_t)a.q & qmask) == 0 &&
+      ((uintptr_t)a.out & 15) == 0 && (DqTraits<F>::BLOCK || a.group >= 8)) {
     a.div = fast_div((uint32_t)(DqTraits<F>::BLOCK ? a.N / 8 : a.group));
     const int64_t nb = (n / 8 + DQ_THREADS * DQ_U - 1) / (DQ_THREADS * DQ_U);
     hipLaunchKernelGGL((k_dequant<F, DT>), dim3((unsigned)(nb > 0 ? nb : 1)), dim3(DQ_THREADS), 0, st, a);

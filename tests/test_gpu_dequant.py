@@ -137,3 +137,18 @@ def test_mx(shape: tuple[int, int], elem: torch.dtype, swizzled: bool, dtype: to
         want = O.mx_dequant(q, s, fmt, cols, swizzled=swizzled, cd=OUT[dtype])
     for off in (False, True):
         _check(K.dequantize_mx(_dev(q, off), _dev(s), elem, cols, swizzled=swizzled, dtype=dtype), want, dtype)
+
+
+def test_swizzled_scale_offsets_beyond_32_bits() -> None:
+    """One row of more than 2^29 columns: its swizzled scales are padded to 128 rows, 2^32 bytes and 512 more.  The last
+    block's scales sit past 2^32, where an offset of 32 bits would read the first block's."""
+    cols = (1 << 29) + 64
+    q = torch.full((1, cols // 2), 0x22, dtype=torch.uint8, device="cuda")  # every code is 1.0
+    s = torch.full((32, cols // 64 * 16), 0x38, dtype=torch.uint8, device="cuda")  # 1.0
+    assert s.numel() == (1 << 32) + 512
+    s.view(-1)[:4] = 0x30  # 0.5
+    s.view(-1)[1 << 32:(1 << 32) + 4] = 0x40  # 2.0
+    got = K.dequantize_nvfp4(q, s.view(torch.float8_e4m3fn), None, swizzled=True)[0]
+    assert torch.equal(got[-64:].cpu(), torch.full((64,), 2.0, dtype=torch.bfloat16))
+    assert torch.equal(got[:64].cpu(), torch.full((64,), 0.5, dtype=torch.bfloat16))
+    assert bool((got[64:-64] == 1).all())
