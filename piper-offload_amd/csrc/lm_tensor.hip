@@ -142,19 +142,29 @@ int pass(const RowArgs& a, int& npart, hipStream_t st) {
   LAUNCH_CHECK();
   return LM_OK;
 }
-// Wave tiles, amax and quant pass (us per call, FP8).  Rank <= 32: 4 row
-// blocks x 8 tiles and 2 x 4: [13800, 5120] rank 32 61.8 ((4, 4) and (2, 4):
-// 62.9, (2, 4) and (2, 4): 67.1, (8, 8) and (4, 8): 68.4).  Rank 64, whose
-// operands cost more per tile: (8, 8) and (4, 8) [8192, 8192] 73.0 ((8, 4) and
-// (4, 4): 75.8, (4, 8) and (2, 4): 88.3), but those leave smaller weights with
-// less than a wave per SIMD ((8, 8) and (4, 8): [4096, 4096] 33.0 against 25.8).
+// Wave tiles (row blocks x tiles), amax and quant pass; us per call, FP8.
+// Below 2^23 elements the larger tiles leave SIMDs without a wave: 2 x 1 for
+// both passes ([1024, 4096] rank 32 11.9, rank 64 16.4; with the tiles that
+// follow 19.9 and 31.5; k_blocks 22.6 and 27.7; [2000, 4096] rank 64 24.0
+// against 32.1), unless a row has fewer than 4 tiles, so that only row
+// blocks share operands.  Above, rank <= 32: 4 x 8 and 2 x 4 ([13800, 5120]
+// rank 32 57.8 with 4 x 8 and 4 x 8 57.6, 4 x 4 and 2 x 4 59.7, 2 x 4 and 2 x 4
+// 63.3).  Rank 64, whose operands cost more per tile: 8 x 4 and 4 x 4, from 2^26
+// elements on 8 x 8 and 4 x 8.  The lines, rank 64: the first pair and the
+// second, [4096, 6144] 42.8 and 52, [4096, 11008] 62 and 67, [4096, 14336] 72.3
+// and 68.2, [8192, 8192] 72.4 and 67.9, [13800, 5120] 91 and 91.
 template <int KIND, bool SR, int NKC>
 int run(const RowArgs& a, hipStream_t st) {
   int npart = 0, rc;
+  const int64_t n = a.M * a.N;
+  if (n < (INT64_C(1) << 23) && a.N >= 64 * TT_NW) {
+    rc = pass<KIND, false, NKC, 2, 1, false>(a, npart, st);
+    return rc ? rc : pass<KIND, SR, NKC, 2, 1, true>(a, npart, st);
+  }
   if constexpr (NKC < 4) {
     rc = pass<KIND, false, NKC, 4, 8, false>(a, npart, st);
     return rc ? rc : pass<KIND, SR, NKC, 2, 4, true>(a, npart, st);
-  } else if (a.M * a.N >= (INT64_C(1) << 26)) {  // 1024 waves of 128 rows x 512 columns
+  } else if (n >= (INT64_C(1) << 26)) {
     rc = pass<KIND, false, NKC, 8, 8, false>(a, npart, st);
     return rc ? rc : pass<KIND, SR, NKC, 4, 8, true>(a, npart, st);
   } else {

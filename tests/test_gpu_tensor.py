@@ -1,6 +1,6 @@
 """Per-tensor FP8 and INT8 merges through csrc/lm_tensor.hip against the oracle's requant of the GPU's dense merge, bit for
-bit and in place: ragged rows, column counts that leave waves without tiles, every rank bucket and both wave tilings of
-rank 64, a weight too short for its row length (which the general kernels take), odd columns and fp16 factors (likewise)."""
+bit and in place: ragged rows, column counts that leave waves without tiles, every rank bucket and all wave tilings of
+each, a weight too short for its row length (which the general kernels take), odd columns and fp16 factors (likewise)."""
 
 from __future__ import annotations
 
@@ -78,3 +78,11 @@ def test_symmetric_with_zero_point(shape: tuple[int, int], in_place: bool) -> No
                            out_qdata=out_q, out_scale=out_s, out_zero_point=out_z)
     assert np.array_equal(u8_np(out_q), oq.view(np.uint8))
     assert out_s.item() == os_[0] and out_z.item() == 0
+
+
+@pytest.mark.parametrize("rank", [5, 32, 64])
+@pytest.mark.parametrize("fmt,sr", [("e4m3", True), ("int8", False)])
+@pytest.mark.parametrize("shape", [(130, 65600), (4100, 2112), (2047, 4096), (2048, 4096)])
+def test_from_2_to_the_23rd_elements(shape: tuple[int, int], fmt: str, sr: bool, rank: int) -> None:
+    """The larger wave tiles: ragged rows and column counts, and either side of the line between them and the small ones."""
+    _case(shape, fmt, sr, rank, torch.bfloat16)
