@@ -1673,10 +1673,20 @@ __global__ __launch_bounds__(256) void k_blocks(BlkArgs a) {
     if (threadIdx.x == 0) {
       float x = __builtin_fmaxf(__builtin_fmaxf(sh_red[0][0], sh_red[0][1]), __builtin_fmaxf(sh_red[0][2], sh_red[0][3]));
       float y = __builtin_fmaxf(__builtin_fmaxf(sh_red[1][0], sh_red[1][1]), __builtin_fmaxf(sh_red[1][2], sh_red[1][3]));
-      // non-negative floats order like their bits; a workgroup whose maximum
-      // another has reached skips the atomic (all of them share one line)
-      raise_max(&a.red[0], f2u(x));
-      raise_max(&a.red[1], f2u(y + 0.0f));
+      // non-negative floats order like their bits.  All workgroups' atomics are
+      // on one line and run one by one, so in a large launch a workgroup whose
+      // maximum another has reached skips its own (raise_max); in a small one
+      // the wait for the load costs more.  us per call, plain atomics and
+      // raise_max: FP8 with fp16 factors 112 workgroups 18.9 and 19.4, 256 22.3
+      // and 20.1; INT8 with zero points 256 23.6 and 24.8, 500 33.0 and 30.7,
+      // 3584 134.5 and 80.2.
+      if (gridDim.x >= (F == B_INT8 ? 384 : 256)) {
+        raise_max(&a.red[0], f2u(x));
+        raise_max(&a.red[1], f2u(y + 0.0f));
+      } else {
+        atomicMax(&a.red[0], f2u(x));
+        atomicMax(&a.red[1], f2u(y + 0.0f));
+      }
     }
   }
 }
