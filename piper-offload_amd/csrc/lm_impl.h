@@ -1271,6 +1271,7 @@ struct BlkArgs {
   int asym;
   int64_t group;          // INT8/FP8 qparam group (N or M*N)
   int tpw;                // macro tiles per wave
+  int look;               // P_AMAX: look before the atomics (k_blocks)
 };
 
 template <int F>
@@ -1679,8 +1680,9 @@ __global__ __launch_bounds__(256) void k_blocks(BlkArgs a) {
       // the wait for the load costs more.  us per call, plain atomics and
       // raise_max: FP8 with fp16 factors 112 workgroups 18.9 and 19.4, 256 22.3
       // and 20.1; INT8 with zero points 256 23.6 and 24.8, 500 33.0 and 30.7,
-      // 3584 134.5 and 80.2.
-      if (gridDim.x >= (F == B_INT8 ? 384 : 256)) {
+      // 3584 134.5 and 80.2.  (a.look: the same test on gridDim.x, read from the
+      // dispatch packet, cost INT8 [65536, 64] rank 64 6 us of 45.)
+      if (a.look) {
         raise_max(&a.red[0], f2u(x));
         raise_max(&a.red[1], f2u(y + 0.0f));
       } else {
@@ -1828,13 +1830,15 @@ static int run_blocks_cd(const BlkArgs& a, int cd, hipStream_t st) {
   constexpr int SPAN = BlkTraits<F>::SPAN;
   unsigned nb = blocks_for(a.M, a.N, 4 * SPAN, a.tpw);
   if (nb == 0) return LM_OK;
+  BlkArgs b = a;
+  b.look = nb >= (F == B_INT8 ? 384 : 256);
   TimedLaunch timed(PASS == P_FULL ? "blocks_full" : PASS == P_AMAX ? "blocks_amax" : PASS == P_QUANT ? "blocks_quant"
                                                                                                     : "todense",
                     st);
   if (cd == LM_F16)
-    hipLaunchKernelGGL((k_blocks<F, F16, NKC, SR, PASS>), dim3(nb), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_blocks<F, F16, NKC, SR, PASS>), dim3(nb), dim3(256), 0, st, b);
   else
-    hipLaunchKernelGGL((k_blocks<F, BF16, NKC, SR, PASS>), dim3(nb), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_blocks<F, BF16, NKC, SR, PASS>), dim3(nb), dim3(256), 0, st, b);
   LAUNCH_CHECK();
   return LM_OK;
 }
