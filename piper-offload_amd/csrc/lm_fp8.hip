@@ -60,7 +60,8 @@ static int fp8_merge(const uint8_t* q, const float* scale, uint8_t* q_out, float
 template <int KIND>
 static int fp8_requant(const RqArgs& r, int64_t group, int cd, bool sr, void* ws, hipStream_t st) {
   if (group == r.M * r.N && group != r.N) return run_rq_tensor<KIND>(r, cd, false, sr, ws, st);
-  if (rq_rows_ok(r, group)) return run_rq_rows<KIND>(r, group, cd, false, sr, st);
+  const RqPlan plan = rq_plan(r, group);
+  if (plan != RQ_NONE) return run_rq_rows<KIND>(r, plan, group, cd, false, sr, st);
   RowArgs a = rq_row_args(r);
   if (group != r.N) return run_groups<KIND, true>(a, group, cd, LM_F32, false, sr, 0, st);
   return run_rows<KIND, true>(a, cd, LM_F32, false, sr, 0, st);

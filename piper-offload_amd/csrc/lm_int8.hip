@@ -97,7 +97,8 @@ extern "C" int lm_int8_requant(const void* dense, int32_t dense_dtype, int8_t* q
   r.qmin = reduce_range ? -64 : -128;
   r.qmax = reduce_range ? 63 : 127;
   if (group == M * N && group != N) return run_rq_tensor<K_INT8>(r, dense_dtype, asym, sr, workspace, st);
-  if (rq_rows_ok(r, group)) return run_rq_rows<K_INT8>(r, group, dense_dtype, asym, sr, st);
+  const RqPlan plan = rq_plan(r, group);
+  if (plan != RQ_NONE) return run_rq_rows<K_INT8>(r, plan, group, dense_dtype, asym, sr, st);
   RowArgs a = rq_row_args(r);
   if (group != N) return run_groups<K_INT8, true>(a, group, dense_dtype, scale_dtype, asym, sr, 0, st);
   return run_rows<K_INT8, true>(a, dense_dtype, scale_dtype, asym, sr, 0, st);

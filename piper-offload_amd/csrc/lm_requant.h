@@ -8,9 +8,10 @@
 // wave's load covers contiguous memory, and one Philox call serves a lane's 8
 // elements.  HBM traffic bounds all of them (2 bytes read, 0.5 to 1 written
 // per element), then the requant arithmetic.
-//   k_rq_rows   per-row INT8 / FP8 of 1024 elements and more: a row's values stay in registers (8 chunks
-//               per lane, all requested at once) between the row maximum and
-//               the encode; the waves of a row meet in LDS.
+//   k_rq_rows   per-row INT8 / FP8, except long lists of short rows (rq_plan): a
+//               row's values stay in registers (8 chunks per lane, all requested
+//               at once) between the row maximum and the encode; the waves of a
+//               row meet in LDS.
 //   k_rq_groups per-group INT8 / FP8 with groups (or whole rows) of 16 .. 512
 //               elements, a power of two: the group's lanes reduce with DPP.
 //   k_rq_amax   per-tensor max and min: one partial per workgroup, no atomics
@@ -559,22 +560,25 @@ static int rq_amax_launch(RqArgs& a, void* ws, hipStream_t st) {
     }                                                                                                              \
   } while (0)
 
-// whether the flat kernels take a per-row (group == N) or per-group encode:
-// whole 16-byte chunks per row, and groups of 2 .. 64 lanes (short rows among
-// them) or rows of at least 1024 elements that fit 16 waves' registers.  The
-// MFMA-layout kernels k_rows and k_groups take the rest: odd columns, misaligned
-// storage, groups that are no power of two, and short rows that are none, of
-// which k_rq_rows' waves hold one each.  2^26 elements, FP8 round to nearest, us:
-// rows of 64 k_rq_groups 34.5, k_rq_rows 394, k_rows 173; of 192 k_rq_rows 137,
-// k_rows 70; of 768 45 and 38.6; of 1024 36.1 and 37.1 (stochastic 45 and 53).
-static inline bool rq_rows_ok(const RqArgs& a, int64_t group) {
-  if (!a.aligned || a.N % 8 != 0) return false;
-  if (group >= 16 && group <= 512 && (group & (group - 1)) == 0) return true;
-  return group == a.N && a.N >= 1024 && a.N <= 16 * 64 * 8 * RQ_CPT;
+// Per row (group == N) or per group: the flat kernels need whole 16-byte chunks
+// per row.  k_rq_rows takes rows that fit 16 waves' registers, but rows of less
+// than 1024 elements, of which its waves hold one each, only while they are few
+// enough for 16 waves per CU; longer lists of such rows, and groups, go through
+// k_rq_groups (2 .. 64 lanes).  The MFMA-layout kernels k_rows and k_groups take
+// the rest: odd columns, misaligned storage, groups that are no power of two and
+// long lists of short rows that are none.  us per call, FP8 round to nearest:
+// rows of 64, 2^26 elements k_rq_groups 34.5, k_rq_rows 394, k_rows 173; of 192
+// k_rq_rows 137, k_rows 70; of 768 45 and 38.6; of 1024 36.1 and 37.1; [320, 768]
+// k_rq_rows 2.4, k_rows 3.3; [64, 128] k_rq_rows 2.3, k_rq_groups 3.2.
+enum RqPlan { RQ_ROWS, RQ_GROUPS, RQ_NONE };
+static inline RqPlan rq_plan(const RqArgs& a, int64_t group) {
+  if (!a.aligned || a.N % 8 != 0) return RQ_NONE;
+  if (group == a.N && a.N <= 16 * 64 * 8 * RQ_CPT && (a.N >= 1024 || a.M <= 4096)) return RQ_ROWS;
+  return group >= 16 && group <= 512 && (group & (group - 1)) == 0 ? RQ_GROUPS : RQ_NONE;
 }
 template <int KIND>
-static int run_rq_rows(RqArgs a, int64_t group, int cd, bool asym, bool sr, hipStream_t st) {
-  if (group > 512) {  // whole rows
+static int run_rq_rows(RqArgs a, RqPlan plan, int64_t group, int cd, bool asym, bool sr, hipStream_t st) {
+  if (plan == RQ_ROWS) {
     int wpr = 1;
     while ((int64_t)wpr * 64 * 8 * RQ_CPT < a.N) wpr *= 2;
     a.waves_per_row = wpr;

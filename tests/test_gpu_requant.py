@@ -34,7 +34,7 @@ def _sr(sr: bool) -> tuple[int | None, dict]:
     return (seed, {"sr_mode": O.SR_PHILOX8, "seed": seed}) if sr else (None, {})
 
 
-ROWS = [(5, 8), (300, 16), (70, 64), (5, 200), (9, 512), (4, 1016), (3, 264), (9, 4096), (2, 4104), (2, 8200), (2, 16392), (2, 32776), (1, 65536), (2, 65544), (4, 77)]
+ROWS = [(5, 8), (300, 16), (4500, 16), (70, 64), (4097, 64), (4097, 72), (9, 512), (4, 1016), (3, 264), (9, 4096), (2, 4104), (2, 8200), (2, 16392), (2, 32776), (1, 65536), (2, 65544), (4, 77)]
 
 
 def _blocks(shape: tuple[int, int]) -> list[tuple[tuple[int, int], int]]:
