@@ -428,9 +428,10 @@ DEV uint32_t sr_h_of(const uint32_t (&c)[4], int j) {
   const uint32_t w = ((j >> 1) & 1) ? ~c[j >> 1] : c[j >> 1];
   return (j & 1) ? (w & 0xffffu) : (w >> 16);
 }
-template <int SPAN>
+// (ALIGNED: idx0 is known to be a multiple of 8)
+template <int SPAN, bool ALIGNED = false>
 DEV void sr_bits(uint64_t seed, uint64_t idx0, uint32_t (&h)[SPAN]) {
-  if ((idx0 & 7u) == 0) {
+  if (ALIGNED || (idx0 & 7u) == 0) {
 #pragma unroll
     for (int gi = 0; gi < SPAN / 8; ++gi) {
       uint32_t c[4];

@@ -1398,7 +1398,9 @@ __device__ __forceinline__ void blk_store(const BlkArgs& a, int64_t row, int64_t
   constexpr int SPAN = BlkTraits<F>::SPAN;
   const int64_t N = a.N;
   uint32_t h[SPAN];
-  if constexpr (SR) sr_bits<SPAN>(a.seed, (uint64_t)(row * N + c0), h);
+  // (block formats have whole blocks per row; in MXFP4 the test for it is the
+  // better code: [64, 40000] rank 8 22.6 us with it, 27.8 without)
+  if constexpr (SR) sr_bits<SPAN, F == B_Q8_0>(a.seed, (uint64_t)(row * N + c0), h);
   if constexpr (F == B_NVFP4) {
     float bmax = 0.0f;
 #pragma unroll
