@@ -458,10 +458,13 @@ DEV int nv_find(const NvStackItem* __restrict__ items, int count, int64_t t) {
 // resident workgroups, the long ones last) ended on them: 203 -> 123 us per
 // merge of a layer (round to nearest), 280 -> 151 (stochastic), 218 -> 139
 // (swizzled); 8 layers 677 -> 667 and 889 -> 872.  Only a swizzled stack of
-// many units is better off with whole rows (8 layers, stochastic: 917 us,
-// chunked 928): without staged scales a chunk saves nothing but the tail.
+// many units is better off with whole rows, since without staged scales a chunk
+// saves nothing but the tail.  Whole rows and chunks, us, rank 16 stochastic and
+// rank 64 round to nearest: 3 layers (4032 units) 460 and 394, 690 and 619; 5
+// layers (6720) 654 and 615, 994 and 976; 6 layers (8064) 746 and 721, 1144 and
+// 1155; 8 layers (10752) 911 and 923, 1427 and 1478.
 __host__ __device__ static inline int nv_chunks(int64_t N) { return (int)(((N >> 7) + 4 * NV_NW - 1) / (4 * NV_NW)); }
-constexpr int64_t NV_WHOLE_ROWS = 8 * 512;  // 32-row units from which a swizzled stack keeps whole rows
+constexpr int64_t NV_WHOLE_ROWS = 8192;  // 32-row units from which a swizzled stack keeps whole rows
 
 // Single tensors: blocks are independent once the global scale is known, so a
 // workgroup owns 32 rows x NV_CHUNK macro tiles (blockIdx.y picks the chunk).

@@ -182,7 +182,7 @@ static int nv_stack_fast(const lm_stack_item* items, int32_t count, int32_t swiz
   const size_t prep_bytes = align256((size_t)count * sizeof(PrepItem));
   NvStackItem* h = (NvStackItem*)(table + prep_bytes);
   // two-level items first, then single-level ones; each group numbers its
-  // 16-row units from 0 and gets its own quant launch
+  // units (32 rows x a column chunk) from 0 and gets its own quant launch
   int n_two = 0;
   for (int i = 0; i < count; ++i) n_two += items[i].aux != nullptr ? 1 : 0;
   int64_t tiles[2] = {0, 0};

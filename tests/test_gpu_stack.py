@@ -166,8 +166,9 @@ def _nvfp4_errors(side: str, i: int, q, s, pts, expected) -> list[str]:  # noqa:
 
 @pytest.mark.parametrize("shapes", [[(64, 256), (40, 512), (16, 128), (128, 1024)],  # fast kernels (N % 128 == 0)
                                     [(32, 256), (16, 96)],                           # per-target block kernels
-                                    # plain-layout block scales staged in LDS up to 128 macro tiles per row:
-                                    # the limit itself with ragged row groups, then one item past it
+                                    # column chunks of up to 32 macro tiles (nv_chunks), each staging its block
+                                    # scales in LDS when the layout is plain: 4 full chunks with ragged row
+                                    # groups, then 5 uneven ones
                                     [(40, 16384), (33, 4096), (17, 128)],
                                     [(24, 16512), (40, 256)],
                                     LAYER])                                          # one 8B layer at full size

@@ -21,8 +21,20 @@ SHAPES = [(33, 4224), (64, 128), (17, 14336), (96, 8320), (40, 4096), (1, 12416)
 @pytest.mark.parametrize("swizzled", [False, True])
 @pytest.mark.parametrize("sr", [False, True])
 def test_chunked_rows_equal_single_merges(sr: bool, swizzled: bool, rank: int) -> None:
+    _case(SHAPES, sr, swizzled, rank)
+
+
+@pytest.mark.parametrize("sr", [False, True])
+@pytest.mark.parametrize("rows", [32 * 8187, 32 * 8186])
+def test_swizzled_stacks_of_many_rows(rows: int, sr: bool) -> None:
+    """8192 units of 32 rows keep whole rows (NV_WHOLE_ROWS), one unit less is chunked; the second target has rows of 33
+    tiles, one past a chunk."""
+    _case([(rows, 128), (33, 4224), (65, 128)], sr, True, 16)
+
+
+def _case(shapes: list[tuple[int, int]], sr: bool, swizzled: bool, rank: int) -> None:
     targets, want = [], []
-    for i, (rows, cols) in enumerate(SHAPES):
+    for i, (rows, cols) in enumerate(shapes):
         w = normal_bf16((rows, cols), 0.02, i).cuda()
         q, s, p = K.requantize_nvfp4(w, two_level=i % 3 != 2, swizzled=swizzled)
         b, a = (t.cuda() for t in lora_factors(rows, cols, rank, 100 + i))
@@ -30,6 +42,6 @@ def test_chunked_rows_equal_single_merges(sr: bool, swizzled: bool, rank: int) -
         targets.append(StackTarget(NVFP4Weight(q, s, p, 16, is_swizzled_scales=swizzled), b, a, 0.75, 77 + i))
     merge_nvfp4_stack(targets, stochastic=sr)
     for i, (t, (q, s, p)) in enumerate(zip(targets, want)):
-        assert torch.equal(t.weight.qdata, q), SHAPES[i]
-        assert torch.equal(t.weight.scale.view(torch.uint8), s.view(torch.uint8)), SHAPES[i]
+        assert torch.equal(t.weight.qdata, q), shapes[i]
+        assert torch.equal(t.weight.scale.view(torch.uint8), s.view(torch.uint8)), shapes[i]
         assert p is None or torch.equal(t.weight.per_tensor_scale, p)
