@@ -151,3 +151,29 @@ def test_dense_bf16_merge(shape, rank, strength):
     RegularAdapter.merge_lora_(wd, b.to(DEV), a.to(DEV), strength)
     ref = O.merge_dense(bf16_np(w), bf16_np(b), bf16_np(a), strength)
     assert_merged_close(bf16_np(wd), ref, bf16_np(w))
+
+
+@pytest.mark.parametrize("rank", [5, 32, 64])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(2057, 4104), (33, 200)])
+def test_dense_row_tiles_and_dtypes(shape, dtype, rank):
+    """Waves of two row tiles and of one ([2057, 4104]: 129 tiles for 127 groups), ragged in rows and columns, in both
+    dtypes; a row stride of 16-byte pieces and, for the general kernel, an odd one.  Integer factors make B A exact in
+    every summation order, so results equal the oracle's bit for bit."""
+    rows, cols = shape
+    g = torch.Generator().manual_seed(rows + rank)
+    w = (torch.randn(shape, generator=g) * 4).to(dtype)
+    b = torch.randint(-2, 3, (rows, rank), generator=g).to(dtype)
+    a = torch.randint(-2, 3, (rank, cols), generator=g).to(dtype)
+
+    def bits(t):
+        return t.view(torch.int16).numpy().view(np.uint16)
+
+    dt = O.DT_F16 if dtype is torch.float16 else O.DT_BF16
+    want = torch.from_numpy(O.merge_dense(bits(w), bits(b), bits(a), 0.75, cd=dt, fdt=dt).view(np.int16)).view(dtype)
+    for pad in (0, 8, 3):
+        store = torch.zeros((rows, cols + pad), dtype=dtype, device=DEV)
+        store[:, :cols] = w.to(DEV)
+        K.merge_dense_lora_(store[:, :cols], b.to(DEV), a.to(DEV), 0.75)
+        assert torch.equal(store[:, :cols].cpu().view(torch.int16), want.view(torch.int16))
+        assert not store[:, cols:].any()

@@ -1,6 +1,8 @@
-"""The single-factor up projection in whole cache lines and the down projection's column pairs (csrc/lm_routed.hip): last
-token tiles of 1 to 15 rows, outputs narrower than a tile and of ragged width, input widths that end inside a pair or a
-round, every chunk count.  Same oracle and bounds as test_gpu_routed.py; the output may alias y."""
+"""The routed residual's tilings (csrc/lm_routed.hip), bit for bit against the oracle on inputs whose sums are exact: the
+single-factor up projection in whole cache lines and the down projection's column pairs (last token tiles of 1 to 15 rows,
+outputs narrower than a tile and of ragged width, input widths that end inside a pair or a round, every chunk count), the
+down projection's shares, several token tiles per wave, and an output that aliases y.  test_gpu_routed.py has general
+inputs."""
 
 from __future__ import annotations
 
@@ -9,29 +11,11 @@ import pytest
 import torch
 
 import oracle as O
-import test_gpu_routed
 from piper_offload_amd import _lib as L
 from piper_offload_amd.routed import RoutedFactor, routed_residual
-from test_gpu_routed import DT, _bits, _case, _check
+from test_gpu_routed import DT, _bits
 
 pytestmark = pytest.mark.gpu
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("T,K,N,rank", [(17, 4160, 136, 32), (31, 100, 8, 16), (33, 4104, 72, 64), (129, 8232, 264, 24),
-                                        (24, 36, 64, 4), (47, 1024, 200, 48), (300, 520, 1032, 16)])
-def test_lean_up_matches_oracle(T: int, K: int, N: int, rank: int, dtype: torch.dtype, monkeypatch) -> None:
-    # Elements that may differ at all: a value p = x A^T rounds the other way when its fp32 sum, taken in another order
-    # (about 2^-22 relative apart), lies that close to a rounding boundary: with an ulp of 2^-10 (fp16) or 2^-7 (bf16), one
-    # value in 2^11 or 2^14 or so, and it can move every output of its token.  Four times the expected share of tokens,
-    # plus two tokens (these results have few).
-    share = 4 * rank * 2.0 ** (-11 if dtype is torch.float16 else -14) + 2 / T
-    monkeypatch.setattr(test_gpu_routed, "ROUTED_MISMATCH", max(test_gpu_routed.ROUTED_MISMATCH, share))
-    x, y, fs = _case(T, K, N, [rank], False, dtype, T + K)
-    dfs = [RoutedFactor(f.a.cuda(), f.b.cuda(), f.strength) for f in fs]
-    with torch.no_grad():
-        got = routed_residual(x.cuda(), dfs, y.cuda())
-    _check(got, x, y, fs, dtype)
 
 
 def _integer_case(T: int, K: int, N: int, ranks: list[int], bias: bool, dtype: torch.dtype, seed: int):
@@ -55,6 +39,16 @@ def _oracle(x, y, fs, dtype) -> torch.Tensor:
 
 def _cuda(fs):
     return [RoutedFactor(f.a.cuda(), f.b.cuda(), f.strength, None if f.bias is None else f.bias.cuda()) for f in fs]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,K,N,rank", [(17, 4160, 136, 32), (31, 100, 8, 16), (33, 4104, 72, 64), (129, 8232, 264, 24),
+                                        (24, 36, 64, 4), (47, 1024, 200, 48), (300, 520, 1032, 16)])
+def test_lean_up_matches_oracle(T: int, K: int, N: int, rank: int, dtype: torch.dtype) -> None:
+    x, y, fs = _integer_case(T, K, N, [rank], False, dtype, T + K)
+    with torch.no_grad():
+        got = routed_residual(x.cuda(), _cuda(fs), y.cuda())
+    assert torch.equal(got.cpu(), _oracle(x, y, fs, dtype))
 
 
 # The down projection's shares (down_plan): K spans that end inside a step, chunk blocks of 1, 2 and 4 with a last one of
