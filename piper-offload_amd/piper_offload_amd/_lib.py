@@ -223,5 +223,9 @@ class on_device:
 
 
 def stream_ptr(device: torch.device) -> int:
-    """The raw handle of the device's current stream (without building a ``torch.cuda.Stream``, 3 us)."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    """The raw handle of the device's current stream (without building a ``torch.cuda.Stream``, 3 us).
+
+    A device without an index is the current one, as for ``torch.cuda.current_stream``.
+    """
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

@@ -325,3 +325,12 @@ def test_stack_plan_overlap_check_passes_disjoint_views() -> None:
     a = torch.zeros(16, 64, dtype=torch.bfloat16)
     _reject_shared_buffers([StackTarget(_nv_cpu(32, 64, torch.ones(()), fused[:32]), b, a, 1.0),
                             StackTarget(_nv_cpu(32, 64, torch.ones(()), fused[32:]), b, a, 1.0)])
+
+
+def test_stream_of_a_device_without_an_index_is_the_current_devices(monkeypatch) -> None:
+    from piper_offload_amd import _lib
+
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 1000 + index, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    assert _lib.stream_ptr(torch.device("cuda:5")) == 1005
+    assert _lib.stream_ptr(torch.device("cuda")) == 1003
