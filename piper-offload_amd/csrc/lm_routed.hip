@@ -13,12 +13,12 @@
 //   out    = dt(y + total)
 //
 // At most 16 tokens (decode): one kernel, k_routed_small, and no workspace.
-// Otherwise two or three:
+// Otherwise two (or three):
 // * k_routed_down: MFMA x A^T by 16-wave workgroups whose waves split K and meet
 //   in LDS; writes ps = dt(dt(p) s) in the dtype, [T][C * 16] (C = sum of
 //   ceil(r_i / 16) rank chunks), or, where few tokens leave the GPU idle, the
-//   sums of one of S spans of K (down_plan);
-// * k_routed_finalize (S > 1): adds the spans and writes ps;
+//   sums of one of S spans of K (down_plan), which the up kernel adds itself
+//   (SPANS) or, when they are many, k_routed_finalize;
 // * k_routed_up: a wave keeps the B operands of one 64-column tile in
 //   registers and walks 16-token tiles: one MFMA chain per factor, the rest
 //   of the rounding chain and one read and one write of y / out: the only
@@ -41,6 +41,7 @@ struct RoutedArgs {
   float* part;          // S > 1: [S][T][C * 16], the spans' sums
   int64_t T, K, N;
   int64_t kspan;        // K columns per span of the down projection
+  int S;                // spans
   int nf, nchunks;
   int tiles_per_wg;     // token tiles per up workgroup
   const uint16_t* a[RT_MAX_FACTORS];
@@ -116,7 +117,7 @@ __device__ __forceinline__ v4f32 mfma1(const v4i16& a, const v4i16& b, const v4f
 // (l >> 4) + 0..3 of token l & 15.  The CB chunks share each round's x values;
 // the waves' sums meet in LDS and one thread per (chunk, rank, token) adds them
 // in wave order.  With S = 1 it rounds and writes ps; otherwise it writes the
-// span's partial and k_routed_finalize adds the spans.
+// span's partial.
 constexpr int RT_DNW = 16;
 constexpr int RT_DU = 8;
 constexpr int RT_DSTEP = 64 * RT_DNW;  // columns of one pair per wave: spans are multiples of it
@@ -186,28 +187,29 @@ __global__ __launch_bounds__(RT_DNW * 64) void k_routed_down(RoutedArgs a, FastD
   }
 }
 
-// S > 1: one thread per (token, chunk, 4 ranks) adds the S partials in span
-// order and applies p_i = dt(p), ps_i = dt(p_i s_i)
+// four ranks of ps, two words, from the S partials at p, `stride` floats apart:
+// added in span order, then p_i = dt(p), ps_i = dt(p_i s_i)
+template <int DT>
+__device__ __forceinline__ lm_u32x2 sum_spans(const float* p, int64_t stride, int S, float s) {
+  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+  for (int sp = 0; sp < S; ++sp) {
+    const v4f32 w = *(const LM_GLOBAL v4f32*)(p + sp * stride);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += w[i];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = round_dt<DT>(round_dt<DT>(v[i]) * s);
+  return lm_u32x2{(uint32_t)bits_dt<DT>(v[0]) | ((uint32_t)bits_dt<DT>(v[1]) << 16),
+                  (uint32_t)bits_dt<DT>(v[2]) | ((uint32_t)bits_dt<DT>(v[3]) << 16)};
+}
+// one thread per (token, chunk, 4 ranks)
 template <bool HALF>
-__global__ __launch_bounds__(256) void k_routed_finalize(RoutedArgs a, int S) {
-  constexpr int DT = HALF ? F16 : BF16;
+__global__ __launch_bounds__(256) void k_routed_finalize(RoutedArgs a) {
   const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x, n = a.T * a.nchunks * 4;
   if (q >= n) return;
-  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int sp = 0; sp < S; ++sp) {
-    const float4 w = ((const float4*)a.part)[sp * n + q];
-    v[0] += w.x;
-    v[1] += w.y;
-    v[2] += w.z;
-    v[3] += w.w;
-  }
-  const float s = a.s[a.cfac[(int)(q % (a.nchunks * 4)) >> 2]];
-  uint32_t w[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-    w[h] = (uint32_t)bits_dt<DT>(round_dt<DT>(round_dt<DT>(v[2 * h]) * s)) |
-           ((uint32_t)bits_dt<DT>(round_dt<DT>(round_dt<DT>(v[2 * h + 1]) * s)) << 16);
-  ((uint2*)a.ps)[q] = make_uint2(w[0], w[1]);
+  ((LM_GLOBAL lm_u32x2*)a.ps)[q] =
+      sum_spans<HALF ? F16 : BF16>(a.part + 4 * q, 4 * n, a.S, a.s[a.cfac[(int)(q % (a.nchunks * 4)) >> 2]]);
 }
 
 // Columns of the up kernels: in a 64-column tile lane group g = lane >> 4 holds
@@ -260,7 +262,7 @@ __device__ __forceinline__ void up_store(const RoutedArgs& a, int64_t t, int64_t
 // requested one token tile ahead, after the current tile's own loads, so that
 // waiting for the current tile never waits for the prefetch (loads complete
 // in order).
-template <bool HALF, int CMAX>
+template <bool HALF, int CMAX, bool SPANS>
 __global__ __launch_bounds__(RT_NW * 64) void k_routed_up(RoutedArgs a) {
   constexpr int DT = HALF ? F16 : BF16;
   const int lane = threadIdx.x & 63, wave = wave_index(), rl = lane & 15, g = lane >> 4;
@@ -295,7 +297,13 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up(RoutedArgs a) {
 #pragma unroll
     for (int c = 0; c < CMAX; ++c) {
       pv[c] = (v4i16){0, 0, 0, 0};
-      if (c < a.nchunks && ok) pv[c] = __builtin_bit_cast(v4i16, *(const uint2*)(a.ps + t * rowstride + c * 16 + 4 * g));
+      if (c < a.nchunks && ok) {
+        const int64_t at = t * rowstride + c * 16 + 4 * g;
+        if constexpr (SPANS)
+          pv[c] = __builtin_bit_cast(v4i16, sum_spans<DT>(a.part + at, a.T * rowstride, a.S, a.s[a.cfac[c]]));
+        else
+          pv[c] = __builtin_bit_cast(v4i16, *(const uint2*)(a.ps + at));
+      }
     }
     if (ok && vec) {
       const uint16_t* yr = a.y + t * a.N;
@@ -348,7 +356,7 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up(RoutedArgs a) {
 // addresses are scalar bases that advance by a token tile plus constant 32-bit
 // lane offsets; the loads are unconditional (rows past T and columns past N
 // read valid ones), only the stores are predicated.
-template <bool HALF, int NC>
+template <bool HALF, int NC, bool SPANS>
 __global__ __launch_bounds__(RT_NW * 64) void k_routed_up1(RoutedArgs a) {
   constexpr int DT = HALF ? F16 : BF16;
   const int lane = threadIdx.x & 63, wave = wave_index(), rl = lane & 15, g = lane >> 4;
@@ -384,7 +392,12 @@ __global__ __launch_bounds__(RT_NW * 64) void k_routed_up1(RoutedArgs a) {
     y1 = *(const LM_GLOBAL lm_u32x4*)(yt + (off1 - b1 * 2u * (uint32_t)N));
     const LM_GLOBAL uint8_t* pt = ps + (int64_t)tt * (NC * 512);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) pv[c] = *(const LM_GLOBAL lm_u32x2*)(pt + (offp - bp * (NC * 32u) + 32u * c));
+    for (int c = 0; c < NC; ++c) {
+      if constexpr (SPANS)
+        pv[c] = sum_spans<DT>(a.part + ((int64_t)(16 * tt + rl) - bp) * (NC * 16) + 16 * c + 4 * g, a.T * (NC * 16), a.S, a.s[0]);
+      else
+        pv[c] = *(const LM_GLOBAL lm_u32x2*)(pt + (offp - bp * (NC * 32u) + 32u * c));
+    }
   };
   load(tb);
   for (int tt = tb; tt < te; ++tt) {
@@ -525,18 +538,28 @@ __global__ __launch_bounds__(RT_SNW * 64) void k_routed_small(RoutedArgs a) {
 // How the down projection is shared out: CB rank chunks per workgroup, S spans
 // of K.  A workgroup is bound by the latency of its rounds (about 4 us for 4096
 // columns of one chunk), so up to one per CU each more takes work off the
-// others: chunk blocks (a larger block shares its x) and spans (which cost a
-// launch and S partials of p).  Long spans take the largest block that reaches
+// others: chunk blocks (a larger block shares its x) and spans (whose S partials
+// of p are summed afterwards).  Long spans take the largest block that reaches
 // RT_DWG workgroups with them; where that would take spans of less than 3 steps
 // (3072 columns), smaller blocks come first (1024 tokens, rank 64: K 14336 CB 4
 // and S 4 41.6 us, CB 1 and S 1 45.8; K 4096 27.5 and 27.0).  Per call, K -> 4096,
-// one workgroup per 16 tokens -> this: 17 tokens, rank 16, K 4096 12.5 -> 9.4 us;
-// four rank-64 factors, K 4096 94 -> 26, K 14336 277 -> 30; 256 tokens, rank 64,
-// K 14336 71 -> 20; 1024 tokens, rank 64, K 4096 37.1 -> 26.8.  More than RT_DWG
+// one workgroup per 16 tokens -> this: 17 tokens, rank 16, K 4096 12.5 -> 7.9 us;
+// four rank-64 factors, K 4096 94 -> 28, K 14336 277 -> 29; 256 tokens, rank 64,
+// K 14336 71 -> 19; 1024 tokens, rank 64, K 4096 37.1 -> 27.0.  More than RT_DWG
 // workgroups do not pay (2048 tokens, K 4096: rank 16 20.0 us with 128 or 256,
 // 21.7 with 512; rank 64 43.6 with 256, 48.4 with 512).
 constexpr int64_t RT_DWG = 256;
 constexpr int64_t RT_MAX_S = 16;
+// Who adds the spans: every wave of the up kernel for its own tokens (no third
+// launch, whose host side costs 2.7 us of a call of 19) with at most 3 chunks,
+// each a serial sum ahead of the MFMAs, and up to RT_FOLD KB of partials read in
+// all.  us, K 4096: 17 tokens rank 16 up kernel 8.1, own launch 9.1, one span 12.5;
+// rank 64 14.4, 11.3, 14.6; -> 14336, rank 16: 256 tokens (14336 KB) 12.2, 12.2,
+// 15.3; 512 (28672 KB) 17.9, 16.6, 18.8; 1024 (57344 KB) 23.6, 21.2, 23.2.
+// Otherwise their own launch, or one span where that takes a single round.
+constexpr int RT_FOLD_CHUNKS = 3;
+constexpr int64_t RT_FOLD = 32768;
+constexpr int64_t RT_ROUND = 32 * RT_DNW * RT_DU;  // columns of a round
 struct DownPlan {
   int cb, blocks;
   int64_t S, kspan;
@@ -610,7 +633,13 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
   a.x = (const uint16_t*)x;
   a.y = (const uint16_t*)y;
   a.out = (uint16_t*)out;
-  const DownPlan d = down_plan(T, K, chunks);
+  DownPlan d = down_plan(T, K, chunks);
+  const bool spans = d.S > 1 && chunks <= RT_FOLD_CHUNKS && (N + 63) / 64 * tiles * chunks * d.S <= RT_FOLD;
+  if (d.S > 1 && !spans && K <= RT_ROUND) {
+    d.S = 1;
+    d.kspan = K;
+  }
+  a.S = (int)d.S;
   a.ps = (uint16_t*)workspace;
   a.part = (float*)((uint8_t*)workspace + align256((size_t)T * (size_t)chunks * 16 * sizeof(uint16_t)));
   a.kspan = d.kspan;
@@ -655,31 +684,37 @@ extern "C" int lm_routed_residual(const void* x, const void* y, void* out, int64
   // (32-bit lane offsets of a token tile)
   const bool lean = count == 1 && !a.bias[0] && (N & 7) == 0 && chunks <= 4 && chunks != 3 && N < (INT64_C(1) << 26) &&
                     T < (INT64_C(1) << 31) - 16;
-#define RT_UP(H_)                                                                                    \
-  if (lean && chunks == 1) hipLaunchKernelGGL((k_routed_up1<H_, 1>), ugrid, block, 0, st, a);        \
-  else if (lean && chunks == 2) hipLaunchKernelGGL((k_routed_up1<H_, 2>), ugrid, block, 0, st, a);   \
-  else if (lean) hipLaunchKernelGGL((k_routed_up1<H_, 4>), ugrid, block, 0, st, a);                  \
-  else if (chunks <= 1) hipLaunchKernelGGL((k_routed_up<H_, 1>), ugrid, block, 0, st, a);                \
-  else if (chunks <= 2) hipLaunchKernelGGL((k_routed_up<H_, 2>), ugrid, block, 0, st, a);           \
-  else if (chunks <= 4) hipLaunchKernelGGL((k_routed_up<H_, 4>), ugrid, block, 0, st, a);           \
-  else hipLaunchKernelGGL((k_routed_up<H_, RT_MAX_CHUNKS>), ugrid, block, 0, st, a);
+#define RT_UP(H_)                                                                                           \
+  if (lean && chunks == 1) hipLaunchKernelGGL((k_routed_up1<H_, 1, false>), ugrid, block, 0, st, a);        \
+  else if (lean && chunks == 2) hipLaunchKernelGGL((k_routed_up1<H_, 2, false>), ugrid, block, 0, st, a);   \
+  else if (lean) hipLaunchKernelGGL((k_routed_up1<H_, 4, false>), ugrid, block, 0, st, a);                  \
+  else if (chunks <= 1) hipLaunchKernelGGL((k_routed_up<H_, 1, false>), ugrid, block, 0, st, a);            \
+  else if (chunks <= 2) hipLaunchKernelGGL((k_routed_up<H_, 2, false>), ugrid, block, 0, st, a);            \
+  else if (chunks <= 4) hipLaunchKernelGGL((k_routed_up<H_, 4, false>), ugrid, block, 0, st, a);            \
+  else hipLaunchKernelGGL((k_routed_up<H_, RT_MAX_CHUNKS, false>), ugrid, block, 0, st, a);
+#define RT_UP_SPANS(H_)                                                                                     \
+  if (lean && chunks == 1) hipLaunchKernelGGL((k_routed_up1<H_, 1, true>), ugrid, block, 0, st, a);         \
+  else if (lean && chunks == 2) hipLaunchKernelGGL((k_routed_up1<H_, 2, true>), ugrid, block, 0, st, a);    \
+  else if (chunks <= 1) hipLaunchKernelGGL((k_routed_up<H_, 1, true>), ugrid, block, 0, st, a);             \
+  else if (chunks <= 2) hipLaunchKernelGGL((k_routed_up<H_, 2, true>), ugrid, block, 0, st, a);             \
+  else hipLaunchKernelGGL((k_routed_up<H_, RT_FOLD_CHUNKS, true>), ugrid, block, 0, st, a);
   const FastDiv by_blocks = fast_div((uint32_t)d.blocks);
   const dim3 dgrid((unsigned)(tiles * d.blocks), (unsigned)d.S), dblock(RT_DNW * 64);
   const dim3 fgrid((unsigned)((T * chunks * 4 + 255) / 256));
-#define RT_DOWN(H_)                                                                                  \
+#define RT_RUN(H_)                                                                                      \
   if (d.cb == 1) hipLaunchKernelGGL((k_routed_down<H_, 1>), dgrid, dblock, 0, st, a, by_blocks);        \
   else if (d.cb == 2) hipLaunchKernelGGL((k_routed_down<H_, 2>), dgrid, dblock, 0, st, a, by_blocks);   \
   else hipLaunchKernelGGL((k_routed_down<H_, 4>), dgrid, dblock, 0, st, a, by_blocks);                  \
-  if (d.S > 1) hipLaunchKernelGGL(k_routed_finalize<H_>, fgrid, dim3(256), 0, st, a, (int)d.S);
+  if (d.S > 1 && !spans) hipLaunchKernelGGL(k_routed_finalize<H_>, fgrid, dim3(256), 0, st, a);         \
+  if (spans) { RT_UP_SPANS(H_) } else { RT_UP(H_) }
   if (dtype == LM_F16) {
-    RT_DOWN(true)
-    RT_UP(true)
+    RT_RUN(true)
   } else {
-    RT_DOWN(false)
-    RT_UP(false)
+    RT_RUN(false)
   }
-#undef RT_DOWN
+#undef RT_RUN
 #undef RT_UP
+#undef RT_UP_SPANS
   LAUNCH_CHECK();
   return LM_OK;
 }

@@ -6,7 +6,7 @@ parent module stages the factors on the input's device (cached) and returns
 
     residual = sum_i ((x @ A_i.T) * s_i) @ B_i.T (+ bias_i * s_i)
 
-computed by ``lm_routed_residual``: an MFMA down projection into a small fp32
+computed by ``lm_routed_residual``: an MFMA down projection into a small
 workspace, then one kernel that applies the reference's roundings (every
 step in the output dtype, matmuls accumulated in fp32), multiplies by B and
 adds into a new output, reading and writing the ``[T, N]`` output once.  At

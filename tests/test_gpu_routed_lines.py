@@ -52,13 +52,17 @@ def test_lean_up_matches_oracle(T: int, K: int, N: int, rank: int, dtype: torch.
 
 
 # The down projection's shares (down_plan): K spans that end inside a step, chunk blocks of 1, 2 and 4 with a last one of
-# fewer chunks, one span and many, more tiles than workgroups wanted.
+# fewer chunks, one span and many, more tiles than workgroups wanted; spans summed by a launch of their own and by both up
+# kernels, for one token tile per wave and for two.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,K,N,ranks,bias", [(17, 14336, 72, [64, 64, 64, 64], False), (33, 4100, 200, [16], False),
                                               (130, 3080, 64, [8, 40, 64], True), (300, 9000, 136, [16], False),
                                               (1030, 2056, 72, [64], False), (1024, 7000, 64, [64], False),
                                               (1100, 6200, 40, [48, 16, 5], True), (2050, 1024, 64, [16, 16], False),
-                                              (4100, 256, 64, [64], False), (17, 1024, 64, [1], False)])
+                                              (4100, 256, 64, [64], False), (17, 1024, 64, [1], False),
+                                              (70, 9000, 1000, [16, 8], True), (40, 5000, 100, [16, 16, 9], False),
+                                              (20, 12000, 136, [30], False), (637, 2100, 14336, [16], False),
+                                              (637, 2100, 14336, [8], True)])
 def test_down_projection_shares(T: int, K: int, N: int, ranks: list[int], bias: bool, dtype: torch.dtype) -> None:
     x, y, fs = _integer_case(T, K, N, ranks, bias, dtype, T + K)
     with torch.no_grad():
