@@ -181,7 +181,7 @@ __global__ __launch_bounds__(RT_DNW * 64) void k_routed_down(RoutedArgs a, FastD
 #pragma unroll
       for (int w = 0; w < RT_DNW; ++w) sum += sh[c][w][e];
       const int64_t at = t * (a.nchunks * 16) + (c0 + c) * 16 + 4 * (e >> 6) + (e & 3);
-      if (gridDim.y > 1) a.part[(int64_t)blockIdx.y * a.T * (a.nchunks * 16) + at] = sum;
+      if (a.S > 1) a.part[(int64_t)blockIdx.y * a.T * (a.nchunks * 16) + at] = sum;
       else a.ps[at] = bits_dt<DT>(round_dt<DT>(round_dt<DT>(sum) * a.s[a.cfac[c0 + c]]));
     }
   }
